@@ -84,11 +84,11 @@ struct Ctx {
   // forcing
   double *ft = nullptr, *fm = nullptr, *fq = nullptr;
   // scratch
-  double *cv = nullptr, *ct = nullptr, *cdp = nullptr, *cdiv = nullptr;
-  double *vt_a = nullptr, *tt_a = nullptr, *dpt_a = nullptr, *vt_b = nullptr, *tt_b = nullptr, *dpt_b = nullptr;
+  double *pre[2] = {};   // pre-exchange states [ie][4][sc] (state_chunk)
+  double *cdiv = nullptr;
   double *qdp_pre = nullptr, *qbih = nullptr, *qbih_pre = nullptr, *qlim[2] = {}, *fdss_pre = nullptr;
-  // stage-2 pre-exchange buffers: qdp_pre2 (later qbih) and an alias of ct,
-  // which is free from the stage-2 advection until its exchange has consumed it
+  // stage-2 pre-exchange buffers: qdp_pre2 (later qbih) and an alias of
+  // pre[0], which is free during the tracer step
   double *qdp_pre2 = nullptr, *fdss_pre2 = nullptr;
   int *err_d = nullptr;
   int *err_h = nullptr;
@@ -310,16 +310,9 @@ void alloc_work() {
   const size_t q3 = e3 * (c.qsize ? c.qsize : 1);
   // pre-exchange buffers: whole 8-level chunks per element and field
   const size_t e3c = (size_t)c.nelem * lc_field(c.nlev), q3c = e3c * (c.qsize ? c.qsize : 1);
-  c.cv = dalloc<double>(2 * e3);
-  c.ct = dalloc<double>(e3c > e3 ? e3c : e3);  // also the stage-2 fdss_pre
-  c.cdp = dalloc<double>(e3);
+  const size_t sc = c.nelem * std::max(sc_field<4>(c.nlev), sc_field<6>(c.nlev));
+  for (double *&p : c.pre) p = dalloc<double>(std::max(4 * sc, e3c));
   c.cdiv = dalloc<double>(e3);
-  c.vt_a = dalloc<double>(2 * e3);
-  c.vt_b = dalloc<double>(2 * e3);
-  c.tt_a = dalloc<double>(e3);
-  c.tt_b = dalloc<double>(e3);
-  c.dpt_a = dalloc<double>(e3);
-  c.dpt_b = dalloc<double>(e3);
   // Five 40-F3 tracer uses share two allocations (at Q = 40); no kernel
   // writes the allocation it gathers from:
   //   qdp_pre : stage-1 pre-exchange (-> the stage-2 gather), then the first
@@ -334,7 +327,7 @@ void alloc_work() {
   c.qlim[0] = dalloc<double>((size_t)c.nelem * (c.qsize ? c.qsize : 1) * ql_row(c.nlev));
   c.qlim[1] = dalloc<double>((size_t)c.nelem * (c.qsize ? c.qsize : 1) * ql_row(c.nlev));
   c.fdss_pre = dalloc<double>(e3c);
-  c.fdss_pre2 = c.ct;
+  c.fdss_pre2 = c.pre[0];
   c.err_d = dalloc<int>(1);
   if (!c.err_h) hipHostMalloc((void **)&c.err_h, sizeof(int));
   c.be_set = true;
@@ -346,77 +339,44 @@ struct StateBuf {
   double *v, *t, *dp;
 };
 
-// out = DSS_r( sph*(a + dt*RHS(b)) ): one CAAR stage with its DSS.  lap1:
-// the DSS also forms the first hyperviscosity laplacians of out (FP64 form)
-void caar_run(const StateBuf &sa, const StateBuf &sb, const StateBuf &out, double dt, double eta_ave_w,
-              bool lap1 = false) {
-  Ctx &c = C();
-  CaarArgs a{};
-  a.m = metric();
-  a.nelem = c.nelem;
-  a.nlev = c.nlev;
-  a.qsize = c.qsize;
-  a.v_n0 = sb.v;
-  a.t_n0 = sb.t;
-  a.dp_n0 = sb.dp;
-  a.v_nm1 = sa.v;
-  a.t_nm1 = sa.t;
-  a.dp_nm1 = sa.dp;
-  a.qdp_n0 = (c.p.moist && c.qsize > 0) ? c.qdp[c.n0_qdp] : nullptr;
-  a.vn0 = c.vn0;
-  a.omega = c.omega;
-  a.phi = c.phi;
-  a.divv = c.cdiv;
-  a.rsplit0 = c.p.rsplit == 0;
-  a.hybi = c.hybi_d;
-  a.eta_acc = c.eta_dot;
-  a.out_v = c.cv;
-  a.out_t = c.ct;
-  a.out_dp = c.cdp;
-  a.dt = dt;
-  a.eta_ave_w = eta_ave_w;
-  a.p_top = c.hyai0 * c.ps0;
-  {
-    Scope s("caar");
-    launch_caar(c.st, a);
-  }
-  DssArgs x{};
-  x.nf = 4;
-  x.nelem = c.nelem;
-  x.nlev = c.nlev;
-  x.src = c.dss_src;
-  x.rsmp = c.rspheremp;
-  const long long es = (long long)c.nlev * 16, ev = (long long)c.nlev * 32;
-  x.f[0] = {c.cv, out.v, ev, 32};
-  x.f[1] = {c.cv + 16, out.v + 16, ev, 32};
-  x.f[2] = {c.ct, out.t, es, 16};
-  x.f[3] = {c.cdp, out.dp, es, 16};
-  if (lap1) {
-    x.lap1 = c.form == 1 && c.consthv ? 2 : 1;  // the mixed form's FP32 first laplacians
-    x.m = metric();
-    x.lap_v = c.vt_a;
-    x.lap_t = c.tt_a;
-    x.lap_dp = c.dpt_a;
-    x.nu_ratio1 = c.p.nu_ratio1;
-  }
-  Scope s("caar_dss");
-  launch_dss(c.st, x);
-}
+// The five RK stages (u3_5stage, prim_advance_exp.cpp:113-161).  The state of
+// stage i+1 is u[i]; w = (5 u[1] - u[0])/4, out the result.  keep: u[2..4] are
+// stored too (they may be one buffer otherwise; u[1] and w may be one).
+struct RkBufs {
+  StateBuf u[5], w, out;
+  bool keep = false;
+};
 
 StateBuf level(int tl) {
   Ctx &c = C();
   return {c.v[tl], c.t[tl], c.dp[tl]};
 }
 
-void caar_stage(int nm1, int n0, int np1, double dt, double eta_ave_w, bool lap1 = false) {
-  caar_run(level(nm1), level(n0), level(np1), dt, eta_ave_w, lap1);
+int chunk() {
+  Ctx &c = C();
+  return state_chunk(c.nlev, c.p.rsplit == 0);
 }
 
-// hyperviscosity's first laplacians are formed by the last RK stage's DSS
-// (with at least one subcycle)
-bool hv_lap1_fused() {
+// out = DSS_r(pre); lap1: also its first hyperviscosity laplacians
+void state_dss(const double *pre, const StateBuf &out, bool lap1 = false) {
   Ctx &c = C();
-  return c.p.hypervis_subcycle > 0;
+  StateDssArgs x{};
+  x.m = metric();
+  x.src = c.dss_src;
+  x.nelem = c.nelem;
+  x.nlev = c.nlev;
+  x.chunk = chunk();
+  x.pre = pre;
+  x.v = out.v;
+  x.t = out.t;
+  x.dp = out.dp;
+  if (lap1) {
+    x.lap1 = c.form == 1 && c.consthv ? 2 : 1;  // the mixed form's FP32 first laplacians
+    x.lap = c.pre[1];
+    x.nu_ratio1 = c.p.nu_ratio1;
+  }
+  Scope s("caar_dss");
+  launch_state_dss(c.st, x);
 }
 
 bool stop_here(int phase) {
@@ -425,36 +385,92 @@ bool stop_here(int phase) {
   return c.stopped;
 }
 
-void u3_5stage(int nm1, int n0, int np1, double dt, double eta_ave_w) {
+void rk_stages(const RkBufs &r, double dt, double eta_ave_w) {
   Ctx &c = C();
-  caar_stage(n0, n0, nm1, dt / 5.0, eta_ave_w / 4.0);
-  if (stop_here(1)) return;
-  caar_stage(n0, nm1, np1, dt / 5.0, 0.0);
-  caar_stage(n0, np1, np1, dt / 3.0, 0.0);
-  caar_stage(n0, np1, np1, 2.0 * dt / 3.0, 0.0);
-  {
-    Scope s("rk_combo");
-    launch_rk_combo(c.st, c.nelem, c.nlev, c.v[nm1], c.t[nm1], c.dp[nm1], c.v[n0], c.t[n0], c.dp[n0]);
+  // rsplit > 0: each stage gathers the one before it; the vertical advection
+  // of rsplit == 0 reads neighbour levels, so its stages read stored states
+  const bool gather = c.p.rsplit > 0;
+  const double h[5] = {dt / 5.0, dt / 5.0, dt / 3.0, 2.0 * dt / 3.0, 3.0 * dt / 4.0};
+  const double eta[5] = {eta_ave_w / 4.0, 0.0, 0.0, 0.0, 3.0 * eta_ave_w / 4.0};
+  for (int i = 0; i < 5; ++i) {
+    CaarArgs a{};
+    a.m = metric();
+    a.src = c.dss_src;
+    a.nelem = c.nelem;
+    a.nlev = c.nlev;
+    a.qsize = c.qsize;
+    a.chunk = chunk();
+    if (i > 0 && gather) {
+      a.pre = c.pre[(i - 1) & 1];
+      if (i == 1 || r.keep) {
+        a.out_v = r.u[i].v;
+        a.out_t = r.u[i].t;
+        a.out_dp = r.u[i].dp;
+      }
+    } else {
+      a.v = r.u[i].v;
+      a.t = r.u[i].t;
+      a.dp = r.u[i].dp;
+    }
+    if (i > 0) {
+      a.bv = r.u[0].v;
+      a.bt = r.u[0].t;
+      a.bdp = r.u[0].dp;
+    }
+    if (i == 4) {
+      a.u1v = r.u[1].v;
+      a.u1t = r.u[1].t;
+      a.u1dp = r.u[1].dp;
+      a.wv = r.w.v;
+      a.wt = r.w.t;
+      a.wdp = r.w.dp;
+    }
+    a.qdp_n0 = (c.p.moist && c.qsize > 0) ? c.qdp[c.n0_qdp] : nullptr;
+    a.vn0 = c.vn0;
+    a.omega = c.omega;
+    a.rsplit0 = c.p.rsplit == 0;
+    a.hybi = c.hybi_d;
+    a.eta_acc = c.eta_dot;
+    a.pre_out = c.pre[i & 1];
+    a.dt = h[i];
+    a.eta_ave_w = eta[i];
+    a.p_top = c.hyai0 * c.ps0;
+    {
+      Scope s("caar");
+      launch_caar(c.st, a);
+    }
+    const bool stop = i == 0 && c.debug_stop == 1;
+    if (i < 4 && (!gather || stop)) state_dss(a.pre_out, r.u[i + 1]);
+    if (stop && stop_here(1)) return;
   }
-  caar_stage(nm1, np1, np1, 3.0 * dt / 4.0, 3.0 * eta_ave_w / 4.0, hv_lap1_fused());
+  state_dss(c.pre[0], r.out, true);
 }
 
-HvArgs hv_args(const StateBuf &x, double dt, double eta_ave_w) {
+void u3_5stage(int nm1, int n0, int np1, double dt, double eta_ave_w) {
+  RkBufs r;
+  r.u[0] = level(n0);
+  r.u[1] = r.w = level(nm1);
+  r.u[2] = r.u[3] = r.u[4] = r.out = level(np1);
+  rk_stages(r, dt, eta_ave_w);
+}
+
+// one subcycle of hyperviscosity from the state x to o
+HvArgs hv_args(const StateBuf &x, const StateBuf &o, double dt, double eta_ave_w) {
   Ctx &c = C();
   HvArgs a{};
   a.m = metric();
   a.src = c.dss_src;
   a.nelem = c.nelem;
   a.nlev = c.nlev;
+  a.chunk = chunk();
   a.v = x.v;
   a.t = x.t;
   a.dp = x.dp;
-  a.vt_a = c.vt_a;
-  a.tt_a = c.tt_a;
-  a.dpt_a = c.dpt_a;
-  a.vt_b = c.vt_b;
-  a.tt_b = c.tt_b;
-  a.dpt_b = c.dpt_b;
+  a.vo = o.v;
+  a.to = o.t;
+  a.dpo = o.dp;
+  a.lap = c.pre[1];  // where state_dss leaves the first laplacians
+  a.pre = c.pre[0];
   a.dpdiss_ave = c.dpdiss_ave;
   a.dpdiss_bih = c.dpdiss_bih;
   a.dt = dt / c.p.hypervis_subcycle;
@@ -474,12 +490,11 @@ HvArgs hv_args(const StateBuf &x, double dt, double eta_ave_w) {
 
 void hyperviscosity(int np1, double dt, double eta_ave_w) {
   Ctx &c = C();
-  const HvArgs a = hv_args(level(np1), dt, eta_ave_w);
+  const HvArgs a = hv_args(level(np1), level(np1), dt, eta_ave_w);
   const int nsub = c.p.hypervis_subcycle;
-  const bool first = hv_lap1_fused();  // the first laplacians came with the last RK stage
   for (int cyc = 0; cyc < nsub; ++cyc) {
     Scope s("hv_cycle");
-    launch_hv_cycle(c.st, a, cyc > 0 || first, cyc + 1 < nsub);
+    launch_hv_cycle(c.st, a, cyc + 1 < nsub);
   }
 }
 
@@ -1043,17 +1058,13 @@ void dyn_forward_stages(const StateBuf &x, Stages &s, double dt) {
   const int nsub = c.p.hypervis_subcycle;
   std::vector<StateBuf> &U = s.U, &H = s.H;
   copy_state(U[0], x, f3);
-  caar_run(U[0], U[0], U[1], dt / 5.0, 0.0);
-  caar_run(U[0], U[1], U[2], dt / 5.0, 0.0);
-  caar_run(U[0], U[2], U[3], dt / 3.0, 0.0);
-  caar_run(U[0], U[3], U[4], 2.0 * dt / 3.0, 0.0);
-  copy_state(s.W, U[1], f3);
-  launch_rk_combo(c.st, c.nelem, c.nlev, s.W.v, s.W.t, s.W.dp, U[0].v, U[0].t, U[0].dp);
-  caar_run(s.W, U[4], H[0], 3.0 * dt / 4.0, 0.0);
-  for (int cyc = 0; cyc < nsub; ++cyc) {
-    copy_state(H[cyc + 1], H[cyc], f3);
-    launch_hv_cycle(c.st, hv_args(H[cyc + 1], dt, 0.0));
-  }
+  RkBufs r;
+  for (int i = 0; i < 5; ++i) r.u[i] = U[i];
+  r.w = s.W;
+  r.out = H[0];
+  r.keep = true;
+  rk_stages(r, dt, 0.0);
+  for (int cyc = 0; cyc < nsub; ++cyc) launch_hv_cycle(c.st, hv_args(H[cyc], H[cyc + 1], dt, 0.0), cyc + 1 < nsub);
 }
 
 void adj_dyn_forward(AdjBufs &b, int i, double dt) { dyn_forward_stages(b.X[i], b.cur, dt); }

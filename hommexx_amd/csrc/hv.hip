@@ -1,289 +1,312 @@
 // Biharmonic hyperviscosity on the np1 state, one subcycle per call
 // (HyperviscosityFunctorImpl.cpp:56-112, HyperviscosityFunctorImpl.hpp:71-257).
-// Slab kernels: a 16-lane group = one element at one level.
-//   lap1      : weak laplacians of T, dp3d and the vector laplacian of v
-//   DSS(*rsmp)
-//   lap2+pre  : second laplacians, dpdiss accumulators, -nu scaling, the
-//               nu_top sponge on the top three levels, dptens <- dp3d*sph + dt*dptens
-//   DSS + update : assemble, apply the inverse mass, v += , T += - heating/cp,
-//                  dp3d = dptens*rsmp
-// The mixed form swaps in FP32 laplacian kernels (below) and an FP32 first
-// exchange; the second exchange and the update are the same.
+//   lap1      : weak laplacians of T, dp3d and the vector laplacian of v, formed
+//               where the state is assembled: by the exchange of the last RK
+//               stage (state_dss_kernel) and by the previous subcycle's update
+//   lap2      : their exchange (gathered), second laplacians, dpdiss
+//               accumulators, -nu scaling, the nu_top sponge on the top three
+//               levels, dptens <- dp3d*sph + dt*dptens
+//   update    : the exchange of those (gathered), inverse mass, v += ,
+//               T += - heating/cp, dp3d = dptens*rsmp
+// A lane holds one point's chunk of C levels (layout sc_field); the exchanged
+// buffers go back and forth between a.lap and a.pre.  The mixed form forms the
+// laplacians in FP32 and exchanges FP32 first laplacians (summed in FP64).
+//
+// The kernels finish one field before the next (pin), so that a field's C
+// levels of gathers are in flight together and the metric is shared by them.
+// Bound: memory, 30 fields per subcycle at 3.9 TB/s.  One lane per level on the
+// [lev][pt] layout ran at 2.5 to 2.9 TB/s, because each neighbour's edge cost
+// whole 128-byte lines of L2 traffic: three subcycles at ne30 L72 took 1.69 ms
+// then and 1.16 ms now, and the exchange before them 275 and 183 us.  Caps of 3
+// and 4 waves per SIMD spill: 1.58 and 2.41 ms.
 #include "kernels.hpp"
 
 namespace hx {
 
-__device__ __forceinline__ bool slab_of(int nblk, int nelem, int nlev, int &ie, int &k, int &pt) {
-  const int b = xcd_block(blockIdx.x, nblk);
-  const size_t slab = (size_t)b * 16 + (threadIdx.x >> 4);
-  pt = threadIdx.x & 15;
-  if (slab >= (size_t)nelem * nlev) return false;
-  ie = (int)(slab / nlev);
-  k = (int)(slab % nlev);
-  return true;
-}
-
-__global__ __launch_bounds__(256) void hv_lap1_kernel(HvArgs a) {
-  int ie, k, pt;
-  if (!slab_of(gridDim.x, a.nelem, a.nlev, ie, k, pt)) return;
-  const size_t s = ((size_t)ie * a.nlev + k) * 16 + pt;
-  const size_t v = ((size_t)ie * a.nlev + k) * 32 + pt;
-  hv_first_laplacians<false>(a.m, ie, pt, a.nu_ratio1, a.t[s], a.dp[s], a.v[v], a.v[v + 16], a.tt_a, a.dpt_a, a.vt_a,
-                             s, v);
-}
-
-// The first exchange is fused in: each lane gathers the assembled first
-// laplacian of its point (own value and neighbour copies of the vt_a, tt_a,
-// dpt_a outputs of hv_lap1, in dss_kernel's order, times rspheremp) and the
-// outputs go to vt_b, tt_b, dpt_b, which hv_dss_update then exchanges (the
-// inputs of a neighbour's gather are never overwritten during the launch).
-// Slabs are walked in level groups (group_slab) so neighbour copies come
-// from L2.
-// TOP: the nu_top sponge levels 0..2 only (a launch of their own, so that the
-// sponge's extra laplacians do not raise the register count of the main
-// launch: 123 VGPRs without them, 152 with); !TOP with nu_top > 0 skips them.
-template <bool TENSOR, bool TOP>
-__global__ __launch_bounds__(256) void hv_lap2_pre_kernel(HvArgs a) {
-  int ie, k, pt;
-  if (!group_slab(a.nelem, TOP ? (a.nlev < 3 ? a.nlev : 3) : a.nlev, ie, k, pt)) return;
-  if (!TOP && a.nu_top > 0 && k < 3) return;  // whole slab
-  const size_t s = ((size_t)ie * a.nlev + k) * 16 + pt;
-  const size_t v = ((size_t)ie * a.nlev + k) * 32 + pt;
-  double g[4];  // assembled vt (2 components), tt, dpt
-  {
-    const int *src = a.src + ((size_t)ie * 16 + pt) * 3;
-    const int s0 = src[0], s1 = src[1], s2 = src[2];
-    const size_t es = (size_t)a.nlev * 16, ev = (size_t)a.nlev * 32;
-    auto ld = [&](const double *f, size_t estr, size_t lstr, size_t c, double (&r)[4]) {
-      const size_t off = (size_t)k * lstr + c, own = (size_t)ie * estr + off + pt;
-      auto at = [&](int sr) { return opaque_index(sr >= 0 ? (size_t)(sr >> 4) * estr + off + (sr & 15) : own); };
-      r[0] = f[own];
-      r[1] = f[at(s0)];
-      r[2] = f[at(s1)];
-      r[3] = f[at(s2)];
-    };
-    double r0[4], r1[4], rt[4], rdp[4];
-    ld(a.vt_a, ev, 32, 0, r0);
-    ld(a.vt_a, ev, 32, 16, r1);
-    ld(a.tt_a, es, 16, 0, rt);
-    ld(a.dpt_a, es, 16, 0, rdp);
-    const double rs = a.m.rspheremp[(size_t)ie * 16 + pt];
-    g[0] = gather_sum(r0, s0, s1, s2) * rs;
-    g[1] = gather_sum(r1, s0, s1, s2) * rs;
-    g[2] = gather_sum(rt, s0, s1, s2) * rs;
-    g[3] = gather_sum(rdp, s0, s1, s2) * rs;
-  }
+// ------------------------------------------------------------- operators
+// the laplacians of the FP64 and the mixed form on a chunk of levels; P: the
+// type the first laplacians are stored in
+template <bool F32>
+struct HvOps {
+  typedef double P;
   ElemLane e;
-  load_elem(a.m, ie, pt, e);
   DvvLane d;
-  load_dvv(a.m.dvv, pt, d);
-  // second laplacian: constant coefficient, or the tensor form
-  // (HyperviscosityFunctorImpl.hpp:88-128), then the pre-exchange scaling
-  // with the nu_top sponge on the top three levels; each field is finished
-  // and stored before the next one starts (fewer live registers)
+  __device__ __forceinline__ HvOps(const MetricPtrs &m, int ie, int pt) {
+    load_elem(m, ie, pt, e);
+    load_dvv(m.dvv, pt, d);
+  }
+  __device__ __forceinline__ double lap(double x) const { return sph_laplace(e, d, x); }
+  __device__ __forceinline__ double lap_state(double x) const { return lap(x); }
+  __device__ __forceinline__ double vlap(double ratio, double u, double w, double &l1) const {
+    double l0;
+    sph_vlaplace_contra(e, d, ratio, u, w, l0, l1);
+    return l0;
+  }
+};
+template <>
+struct HvOps<true> {
+  typedef float P;
+  ElemLaneF e;
+  DvvLaneF d;
+  __device__ __forceinline__ HvOps(const MetricPtrs &m, int ie, int pt) {
+    load_elemf(m, ie, pt, e);
+    load_dvvf(m.dvv, pt, d);
+  }
+  __device__ __forceinline__ float lap(double x) const { return sph_laplacef(e, d, (float)x); }
+  // of a state's T or dp3d: less its slab reference before rounding
+  __device__ __forceinline__ float lap_state(double x) const { return lap(x - slab_ref(x)); }
+  __device__ __forceinline__ float vlap(double ratio, double u, double w, float &l1) const {
+    float l0;
+    sph_vlaplace_contraf(e, d, (float)ratio, (float)u, (float)w, l0, l1);
+    return l0;
+  }
+};
+
+// the first laplacians of a chunk's levels into lap [ie][4][sc]
+template <int C, bool F32>
+__device__ __forceinline__ void lap1_scalar(const HvOps<F32> &o, const double (&x)[C], typename HvOps<F32>::P *lap) {
+  typename HvOps<F32>::P l[C];
+#pragma unroll
+  for (int j = 0; j < C; ++j) l[j] = o.lap_state(x[j]);
+  sc_store(lap, l);
+}
+template <int C, bool F32>
+__device__ __forceinline__ void lap1_vector(const HvOps<F32> &o, double ratio, const double (&u)[C],
+                                            const double (&w)[C], typename HvOps<F32>::P *lap, size_t lf) {
+  typename HvOps<F32>::P l0[C], l1[C];
+#pragma unroll
+  for (int j = 0; j < C; ++j) l0[j] = o.vlap(ratio, u[j], w[j], l1[j]);
+  sc_store(lap, l0);
+  sc_store(lap + lf, l1);
+}
+
+// The exchange of an RK result (u, v, T, dp3d) into the state arrays.  LAP1:
+// with the first laplacians of the assembled state, from registers.
+template <int C, int LAP1>
+__global__ __launch_bounds__(256) void state_dss_kernel(StateDssArgs a) {
+  int ie, k0, pt;
+  if (!sc_lane<C>(a.nelem, a.nlev, ie, k0, pt)) return;
+  const size_t lf = sc_field<C>(a.nlev);
+  const ScGather<double, C> g(a.pre, 4 * lf, ie, pt, k0, a.src);
+  const double r = a.m.rspheremp[(size_t)ie * 16 + pt];
+  const HvOps<LAP1 == 2> o(a.m, ie, pt);
+  typedef typename HvOps<LAP1 == 2>::P P;
+  P *const lap = (P *)a.lap + (size_t)ie * 4 * lf + (size_t)k0 * 16 + pt * C;
+  double *const v = a.v + ((size_t)ie * a.nlev + k0) * 32 + pt;
+  double *const t = a.t + ((size_t)ie * a.nlev + k0) * 16 + pt;
+  double *const dp = a.dp + ((size_t)ie * a.nlev + k0) * 16 + pt;
+  auto put = [&](double *out, int stride, const double (&x)[C]) {
+#pragma unroll
+    for (int j = 0; j < C; ++j)
+      if (k0 + j < a.nlev) out[j * stride] = x[j];
+  };
+  double x[C], y[C];
+  g.field(3 * lf, r, x);
+  put(dp, 16, x);
+  if (LAP1) lap1_scalar<C, LAP1 == 2>(o, x, lap + 3 * lf);
+  g.field(2 * lf, r, x);
+  put(t, 16, x);
+  if (LAP1) lap1_scalar<C, LAP1 == 2>(o, x, lap + 2 * lf);
+  g.field(0, r, x);
+  g.field(lf, r, y);
+  put(v, 32, x);
+  put(v + 16, 32, y);
+  if (LAP1) lap1_vector<C, LAP1 == 2>(o, a.nu_ratio1, x, y, lap, lf);
+}
+
+template <int C>
+static void launch_state_dss_c(hipStream_t st, const StateDssArgs &a) {
+  const dim3 g(sc_blocks<C>(a.nelem, a.nlev));
+  if (a.lap1 == 2) hipLaunchKernelGGL((state_dss_kernel<C, 2>), g, dim3(256), 0, st, a);
+  else if (a.lap1) hipLaunchKernelGGL((state_dss_kernel<C, 1>), g, dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((state_dss_kernel<C, 0>), g, dim3(256), 0, st, a);
+}
+
+void launch_state_dss(hipStream_t st, const StateDssArgs &a) {
+  if (a.chunk == 6) launch_state_dss_c<6>(st, a);
+  else launch_state_dss_c<4>(st, a);
+}
+
+// Second laplacians: constant coefficient, or (TENSOR) the tensor form
+// (HyperviscosityFunctorImpl.hpp:88-128), and the pre-exchange scaling.  The
+// sponge's laplacians of the state at the top three levels are the element's
+// own first laplacians, read from a.lap; RATIO: except the vector one, where
+// the first laplacian scales the divergence (nu_div != nu).
+template <int C, bool F32, bool TENSOR, bool RATIO>
+__global__ __launch_bounds__(256) void hv_lap2_kernel(HvArgs a) {
+  int ie, k0, pt;
+  if (!sc_lane<C>(a.nelem, a.nlev, ie, k0, pt)) return;
+  typedef typename HvOps<F32>::P P;
+  const int L = a.nlev;
+  const size_t lf = sc_field<C>(L);
+  const ScGather<P, C> g((const P *)a.lap, 4 * lf, ie, pt, k0, a.src);
+  const double rs = a.m.rspheremp[(size_t)ie * 16 + pt];
+  const double sph = a.m.spheremp[(size_t)ie * 16 + pt];
+  const HvOps<F32> o(a.m, ie, pt);
   double tv[4], vs[6];
   if (TENSOR) load_tensor(a.m, ie, pt, tv, vs);
-  const bool top = TOP;  // (the TOP launch runs only with nu_top > 0)
-  const double sc = (k == 0 ? 4.0 : k == 1 ? 2.0 : 1.0) * a.nu_top;
-  {
-    double vt0, vt1;
-    if (TENSOR) sph_vlaplace_cartesian(e, d, tv, vs, g[0], g[1], vt0, vt1);
-    else sph_vlaplace_contra(e, d, a.nu_ratio2, g[0], g[1], vt0, vt1);
-    vt0 *= -a.nu;
-    vt1 *= -a.nu;
-    if (top) {
-      double lv0, lv1;
-      sph_vlaplace_contra(e, d, 1.0, a.v[v], a.v[v + 16], lv0, lv1);
-      vt0 += sc * lv0;
-      vt1 += sc * lv1;
-    }
-    a.vt_b[v] = vt0;
-    a.vt_b[v + 16] = vt1;
-  }
-  {
-    double tt = TENSOR ? sph_laplace_tensor(e, d, tv, g[2]) : sph_laplace(e, d, g[2]);
-    tt *= -a.nu_s;
-    if (top) tt += sc * sph_laplace(e, d, a.t[s]);
-    a.tt_b[s] = tt;
-  }
-  const double dpn = a.dp[s];
-  double dpt = TENSOR ? sph_laplace_tensor(e, d, tv, g[3]) : sph_laplace(e, d, g[3]);
-  a.dpdiss_ave[s] += a.eta_ave_w * dpn / a.nsub;
-  a.dpdiss_bih[s] += a.eta_ave_w * dpt / a.nsub;
-  dpt *= -a.nu_p;
-  if (top) dpt += sc * sph_laplace(e, d, dpn);
-  dpt *= a.dt;
-  dpt += dpn * e.sph;
-  a.dpt_b[s] = dpt;
-}
-
-// ---------------------------------------------------------- mixed form
-// The two laplacians in FP32 (compensated contractions).  The first
-// laplacian's outputs and their assembled values are FP32 arrays held in the
-// first halves of vt_a/tt_a/dpt_a and vt_b/tt_b/dpt_b; T and dp3d are shifted
-// by a per-slab reference value before rounding (laplacians annihilate
-// constants).  Accumulators, scaling, the sponge combination and everything
-// after stay FP64.
-__global__ __launch_bounds__(256) void hv_lap1_mixed_kernel(HvArgs a) {
-  int ie, k, pt;
-  if (!slab_of(gridDim.x, a.nelem, a.nlev, ie, k, pt)) return;
-  const size_t s = ((size_t)ie * a.nlev + k) * 16 + pt;
-  const size_t v = ((size_t)ie * a.nlev + k) * 32 + pt;
-  hv_first_laplacians<true>(a.m, ie, pt, a.nu_ratio1, a.t[s], a.dp[s], a.v[v], a.v[v + 16], a.tt_a, a.dpt_a, a.vt_a,
-                            s, v);
-}
-
-// As hv_lap2_pre: the first exchange of the FP32 first laplacian is gathered
-// here (summed in FP64, times rspheremp, rounded to FP32 like the exchanged
-// array) and the outputs go to the _b buffers.
-__global__ __launch_bounds__(256) void hv_lap2_pre_mixed_kernel(HvArgs a) {
-  int ie, k, pt;
-  if (!group_slab(a.nelem, a.nlev, ie, k, pt)) return;
-  const size_t s = ((size_t)ie * a.nlev + k) * 16 + pt;
-  const size_t v = ((size_t)ie * a.nlev + k) * 32 + pt;
-  float g[4];  // assembled vt (2 components), tt, dpt
-  {
-    const int *src = a.src + ((size_t)ie * 16 + pt) * 3;
-    const int s0 = src[0], s1 = src[1], s2 = src[2];
-    const size_t es = (size_t)a.nlev * 16, ev = (size_t)a.nlev * 32;
-    auto ld = [&](const double *fd, size_t estr, size_t lstr, size_t c, float (&r)[4]) {
-      const float *f = (const float *)fd;
-      const size_t off = (size_t)k * lstr + c, own = (size_t)ie * estr + off + pt;
-      auto at = [&](int sr) { return opaque_index(sr >= 0 ? (size_t)(sr >> 4) * estr + off + (sr & 15) : own); };
-      r[0] = f[own];
-      r[1] = f[at(s0)];
-      r[2] = f[at(s1)];
-      r[3] = f[at(s2)];
-    };
-    float r0[4], r1[4], rt[4], rdp[4];
-    ld(a.vt_a, ev, 32, 0, r0);
-    ld(a.vt_a, ev, 32, 16, r1);
-    ld(a.tt_a, es, 16, 0, rt);
-    ld(a.dpt_a, es, 16, 0, rdp);
-    const double rs = a.m.rspheremp[(size_t)ie * 16 + pt];
-    g[0] = (float)(gather_sum(r0, s0, s1, s2) * rs);
-    g[1] = (float)(gather_sum(r1, s0, s1, s2) * rs);
-    g[2] = (float)(gather_sum(rt, s0, s1, s2) * rs);
-    g[3] = (float)(gather_sum(rdp, s0, s1, s2) * rs);
-  }
-  ElemLaneF e;
-  load_elemf(a.m, ie, pt, e);
-  DvvLaneF d;
-  load_dvvf(a.m.dvv, pt, d);
-  const double sph = a.m.spheremp[(size_t)ie * 16 + pt];
-  double tt = sph_laplacef(e, d, g[2]);
-  double dpt = sph_laplacef(e, d, g[3]);
-  float f0, f1;
-  sph_vlaplace_contraf(e, d, (float)a.nu_ratio2, g[0], g[1], f0, f1);
-  double vt0 = f0, vt1 = f1;
-  const double dpn = a.dp[s];
-  a.dpdiss_ave[s] += a.eta_ave_w * dpn / a.nsub;
-  a.dpdiss_bih[s] += a.eta_ave_w * dpt / a.nsub;
-  double lv0 = 0, lv1 = 0, lt = 0, ldp = 0;
-  const bool top = a.nu_top > 0 && k < 3;
-  if (top) {
-    float g0, g1;
-    sph_vlaplace_contraf(e, d, 1.f, (float)a.v[v], (float)a.v[v + 16], g0, g1);
-    lv0 = g0;
-    lv1 = g1;
-    const double t = a.t[s];
-    lt = sph_laplacef(e, d, (float)(t - slab_ref(t)));
-    ldp = sph_laplacef(e, d, (float)(dpn - slab_ref(dpn)));
-  }
-  vt0 *= -a.nu;
-  vt1 *= -a.nu;
-  tt *= -a.nu_s;
-  dpt *= -a.nu_p;
-  if (top) {
-    const double sc = (k == 0 ? 4.0 : k == 1 ? 2.0 : 1.0) * a.nu_top;
-    vt0 += sc * lv0;
-    vt1 += sc * lv1;
-    tt += sc * lt;
-    dpt += sc * ldp;
-  }
-  dpt *= a.dt;
-  dpt += dpn * sph;
-  a.vt_b[v] = vt0;
-  a.vt_b[v + 16] = vt1;
-  a.tt_b[s] = tt;
-  a.dpt_b[s] = dpt;
-}
-
-// Second exchange fused with the update: the assembled tensors are used at
-// once by the lane that assembled them (same gather order as dss_kernel).
-// LAP1 (1: FP64, 2: mixed form): the same kernel also forms the first
-// laplacians of the updated state for the next subcycle (what hv_lap1_kernel
-// or hv_lap1_mixed_kernel would compute from the stored values), from the
-// values in registers; they go to vt_b, tt_b, dpt_b, which the caller points
-// at the next subcycle's first-laplacian buffers.
-template <int LAP1>
-__global__ __launch_bounds__(256) void hv_dss_update_kernel(HvArgs a) {
-  int ie, k, pt;
-  if (!group_slab(a.nelem, a.nlev, ie, k, pt)) return;
-  const int *src = a.src + ((size_t)ie * 16 + pt) * 3;
-  const int s0 = src[0], s1 = src[1], s2 = src[2];
-  const size_t es = (size_t)a.nlev * 16, ev = (size_t)a.nlev * 32;
-  // the loads of the four gathers are issued before the first sum
-  auto ld = [&](const double *f, size_t estr, size_t lstr, size_t c, double (&r)[4]) {
-    const size_t off = (size_t)k * lstr + c, own = (size_t)ie * estr + off + pt;
-    auto at = [&](int src) { return opaque_index(src >= 0 ? (size_t)(src >> 4) * estr + off + (src & 15) : own); };
-    r[0] = f[own];
-    r[1] = f[at(s0)];
-    r[2] = f[at(s1)];
-    r[3] = f[at(s2)];
+  auto lap2 = [&](double x) -> double {
+    if constexpr (TENSOR) return sph_laplace_tensor(o.e, o.d, tv, x);
+    else return o.lap(x);
   };
-  double r0[4], r1[4], rt[4], rdp[4];
-  ld(a.vt_a, ev, 32, 0, r0);
-  ld(a.vt_a, ev, 32, 16, r1);
-  ld(a.tt_a, es, 16, 0, rt);
-  ld(a.dpt_a, es, 16, 0, rdp);
-  const double b0 = gather_sum(r0, s0, s1, s2), b1 = gather_sum(r1, s0, s1, s2);
-  const double bt = gather_sum(rt, s0, s1, s2), bdp = gather_sum(rdp, s0, s1, s2);
-  const double r = a.m.rspheremp[(size_t)ie * 16 + pt];
-  const size_t i = ((size_t)ie * a.nlev + k) * 16 + pt;
-  const size_t v0 = ((size_t)ie * a.nlev + k) * 32 + pt, v1 = v0 + 16;
-  const double vt0 = (a.dt * b0 * r);
-  const double vt1 = (a.dt * b1 * r);
-  const double u = a.v[v0] + vt0, w = a.v[v1] + vt1;
-  a.v[v0] = u;
-  a.v[v1] = w;
-  const double tt = (a.dt * bt * r);
-  const double heating = vt0 * u + vt1 * w;
-  const double tn = a.t[i] + tt - heating / CP, dpn = (bdp * r);
-  a.t[i] = tn;
-  a.dp[i] = dpn;
-  if (LAP1) hv_first_laplacians<LAP1 == 2>(a.m, ie, pt, a.nu_ratio1, tn, dpn, u, w, a.tt_b, a.dpt_b, a.vt_b, i, v0);
+  const bool top = a.nu_top > 0 && k0 == 0;
+  // the sponge adds sc(j) * (own first laplacian) at levels 0..2
+  auto sponge = [&](size_t off, double (&x)[C]) {
+    if (!top) return;
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+      if (j < L) x[j] += (j == 0 ? 4.0 : j == 1 ? 2.0 : 1.0) * a.nu_top * (double)g.p[0][off + j];
+  };
+  double *const out = a.pre + (size_t)ie * 4 * lf + (size_t)k0 * 16 + pt * C;
+  double x[C], y[C];
+  // ---------------------------------------------------------------- dp3d
+  {
+    double dpn[C], da[C], db[C];
+    const size_t s = ((size_t)ie * L + k0) * 16 + pt;
+    const bool acc = a.eta_ave_w != 0.0;
+    auto at = [&](int j) { return s + (k0 + j < L ? j : L - 1 - k0) * 16; };
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      dpn[j] = a.dp[at(j)];
+      if (acc && !a.first) {
+        da[j] = a.dpdiss_ave[at(j)];
+        db[j] = a.dpdiss_bih[at(j)];
+      } else {
+        da[j] = db[j] = 0.0;
+      }
+    }
+    g.field(3 * lf, rs, x);
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      x[j] = lap2(x[j]);
+      if (acc && k0 + j < L) {
+        a.dpdiss_ave[s + j * 16] = da[j] + a.eta_ave_w * dpn[j] / a.nsub;
+        a.dpdiss_bih[s + j * 16] = db[j] + a.eta_ave_w * x[j] / a.nsub;
+      }
+      x[j] *= -a.nu_p;
+    }
+    sponge(3 * lf, x);
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      x[j] *= a.dt;
+      x[j] += dpn[j] * sph;
+    }
+    sc_store(out + 3 * lf, x);
+  }
+  // ------------------------------------------------------------------- T
+  g.field(2 * lf, rs, x);
+#pragma unroll
+  for (int j = 0; j < C; ++j) x[j] = -a.nu_s * lap2(x[j]);
+  sponge(2 * lf, x);
+  sc_store(out + 2 * lf, x);
+  // ------------------------------------------------------------------- v
+  g.field(0, rs, x);
+  g.field(lf, rs, y);
+#pragma unroll
+  for (int j = 0; j < C; ++j) {
+    P l1;
+    double l0, m1;
+    if constexpr (TENSOR) {
+      sph_vlaplace_cartesian(o.e, o.d, tv, vs, x[j], y[j], l0, m1);
+    } else {
+      l0 = o.vlap(a.nu_ratio2, x[j], y[j], l1);
+      m1 = l1;
+    }
+    x[j] = l0 * -a.nu;
+    y[j] = m1 * -a.nu;
+  }
+  if (!RATIO) {
+    sponge(0, x);
+    sponge(lf, y);
+  } else if (top) {
+    const size_t v = (size_t)ie * L * 32 + pt;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      if (j >= L) break;
+      P l1;
+      const double l0 = o.vlap(1.0, a.v[v + j * 32], a.v[v + j * 32 + 16], l1);
+      const double sc = (j == 0 ? 4.0 : j == 1 ? 2.0 : 1.0) * a.nu_top;
+      x[j] += sc * l0;
+      y[j] += sc * (double)l1;
+    }
+  }
+  sc_store(out, x);
+  sc_store(out + lf, y);
 }
 
-void launch_hv_cycle(hipStream_t st, const HvArgs &a, bool lap1_done, bool lap1_next) {
-  const size_t nslab = (size_t)a.nelem * a.nlev;
-  const int blocks = (int)((nslab + 15) / 16);
-  const dim3 gg(group_blocks_x(a.nelem, a.nlev));
-  // the first exchange is gathered by hv_lap2_pre, which writes the second
-  // laplacian to the _b buffers; the update exchanges those (and, FP64 form,
-  // may form the next subcycle's first laplacians on the way)
-  if (!lap1_done) {
-    if (a.mixed) hipLaunchKernelGGL(hv_lap1_mixed_kernel, dim3(blocks), dim3(256), 0, st, a);
-    else hipLaunchKernelGGL(hv_lap1_kernel, dim3(blocks), dim3(256), 0, st, a);
+// LAP1: with the first laplacians of the updated state for the next subcycle
+// (1: FP64, 2: mixed form), from registers.
+template <int C, int LAP1>
+__global__ __launch_bounds__(256) void hv_update_kernel(HvArgs a) {
+  int ie, k0, pt;
+  if (!sc_lane<C>(a.nelem, a.nlev, ie, k0, pt)) return;
+  const int L = a.nlev;
+  const size_t lf = sc_field<C>(L);
+  const ScGather<double, C> g(a.pre, 4 * lf, ie, pt, k0, a.src);
+  const double r = a.m.rspheremp[(size_t)ie * 16 + pt];
+  const HvOps<LAP1 == 2> o(a.m, ie, pt);
+  typedef typename HvOps<LAP1 == 2>::P P;
+  P *const lap = (P *)a.lap + (size_t)ie * 4 * lf + (size_t)k0 * 16 + pt * C;
+  const size_t s = ((size_t)ie * L + k0) * 16 + pt, v = ((size_t)ie * L + k0) * 32 + pt;
+  auto lv = [&](int j) { return k0 + j < L ? j : L - 1 - k0; };
+  double x[C], y[C], heat[C];
+  {
+    double u[C], w[C];
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      u[j] = a.v[v + lv(j) * 32];
+      w[j] = a.v[v + lv(j) * 32 + 16];
+    }
+    g.field(0, 1.0, x);
+    g.field(lf, 1.0, y);
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      const double v0 = a.dt * x[j] * r, v1 = a.dt * y[j] * r;
+      u[j] += v0;
+      w[j] += v1;
+      heat[j] = v0 * u[j] + v1 * w[j];
+      if (k0 + j < L) {
+        a.vo[v + j * 32] = u[j];
+        a.vo[v + j * 32 + 16] = w[j];
+      }
+    }
+    if (LAP1) lap1_vector<C, LAP1 == 2>(o, a.nu_ratio1, u, w, lap, lf);
   }
-  if (a.mixed) hipLaunchKernelGGL(hv_lap2_pre_mixed_kernel, gg, dim3(256), 0, st, a);
-  else if (a.consthv) hipLaunchKernelGGL((hv_lap2_pre_kernel<false, false>), gg, dim3(256), 0, st, a);
-  else hipLaunchKernelGGL((hv_lap2_pre_kernel<true, false>), gg, dim3(256), 0, st, a);
-  if (!a.mixed && a.nu_top > 0) {
-    const dim3 gt(group_blocks_x(a.nelem, a.nlev < 3 ? a.nlev : 3));
-    if (a.consthv) hipLaunchKernelGGL((hv_lap2_pre_kernel<false, true>), gt, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((hv_lap2_pre_kernel<true, true>), gt, dim3(256), 0, st, a);
+  {
+    double t[C];
+#pragma unroll
+    for (int j = 0; j < C; ++j) t[j] = a.t[s + lv(j) * 16];
+    g.field(2 * lf, 1.0, x);
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      t[j] = t[j] + a.dt * x[j] * r - heat[j] / CP;
+      if (k0 + j < L) a.to[s + j * 16] = t[j];
+    }
+    if (LAP1) lap1_scalar<C, LAP1 == 2>(o, t, lap + 2 * lf);
   }
-  HvArgs b = a;
-  b.vt_a = a.vt_b;
-  b.tt_a = a.tt_b;
-  b.dpt_a = a.dpt_b;
-  b.vt_b = a.vt_a;
-  b.tt_b = a.tt_a;
-  b.dpt_b = a.dpt_a;
-  if (!lap1_next) hipLaunchKernelGGL(hv_dss_update_kernel<0>, gg, dim3(256), 0, st, b);
-  else if (a.mixed) hipLaunchKernelGGL(hv_dss_update_kernel<2>, gg, dim3(256), 0, st, b);
-  else hipLaunchKernelGGL(hv_dss_update_kernel<1>, gg, dim3(256), 0, st, b);
+  g.field(3 * lf, r, x);
+#pragma unroll
+  for (int j = 0; j < C; ++j)
+    if (k0 + j < L) a.dpo[s + j * 16] = x[j];
+  if (LAP1) lap1_scalar<C, LAP1 == 2>(o, x, lap + 3 * lf);
+}
+
+template <int C>
+static void launch_hv_cycle_c(hipStream_t st, const HvArgs &a, bool lap1_next) {
+  const dim3 g(sc_blocks<C>(a.nelem, a.nlev));
+  auto go = [&](auto *kernel) { hipLaunchKernelGGL(kernel, g, dim3(256), 0, st, a); };
+  const bool ratio = a.nu_top > 0 && a.nu_ratio1 != 1.0;
+  if (a.mixed) go(ratio ? hv_lap2_kernel<C, true, false, true> : hv_lap2_kernel<C, true, false, false>);
+  else if (a.consthv) go(ratio ? hv_lap2_kernel<C, false, false, true> : hv_lap2_kernel<C, false, false, false>);
+  else go(ratio ? hv_lap2_kernel<C, false, true, true> : hv_lap2_kernel<C, false, true, false>);
+  if (!lap1_next) go(hv_update_kernel<C, 0>);
+  else if (a.mixed) go(hv_update_kernel<C, 2>);
+  else go(hv_update_kernel<C, 1>);
+}
+
+void launch_hv_cycle(hipStream_t st, const HvArgs &a, bool lap1_next) {
+  if (a.chunk == 6) launch_hv_cycle_c<6>(st, a, lap1_next);
+  else launch_hv_cycle_c<4>(st, a, lap1_next);
 }
 
 }  // namespace hx

@@ -13,16 +13,40 @@ namespace hx {
 
 struct CaarArgs {
   MetricPtrs m;
-  int nelem, nlev, qsize;
-  const double *v_n0, *t_n0, *dp_n0, *v_nm1, *t_nm1, *dp_nm1;
+  const int *src;                      // DSS source table
+  int nelem, nlev, qsize, chunk;       // chunk: state_chunk
+  // the stage's state: gathered from pre-exchange values [ie][4][sc] (u, v,
+  // T, dp3d), with out_v != nullptr also stored; or (pre == nullptr) read
+  // from v, t, dp
+  const double *pre;
+  double *out_v, *out_t, *out_dp;
+  const double *v, *t, *dp;
+  // what the tendency is added to (nullptr: the stage's state): b, or with w
+  // the combination (5 u1 - b)/4, also stored in w (which may be u1)
+  const double *bv, *bt, *bdp;
+  const double *u1v, *u1t, *u1dp;
+  double *wv, *wt, *wdp;
   const double *qdp_n0;  // moist: tracer block of the n0_qdp level (tracer 0 used), else nullptr
-  double *vn0, *omega, *phi;
-  double *divv;                 // scratch: div(v dp) per level
-  int rsplit0;                  // rsplit == 0: Eulerian vertical advection
+  double *vn0, *omega;
+  int rsplit0;                  // rsplit == 0: Eulerian vertical advection (pre == nullptr)
   const double *hybi;           // nlev+1 interface b coefficients (rsplit == 0)
   double *eta_acc;              // eta_dot_dpdn accumulator (rsplit == 0)
-  double *out_v, *out_t, *out_dp;
+  double *pre_out;              // pre-exchange result [ie][4][sc]
   double dt, eta_ave_w, p_top;  // p_top = hyai(0)*ps0
+};
+
+// The exchange of a state's pre-exchange values: assembled values into the
+// state arrays; lap1 also forms the first hyperviscosity laplacians of the
+// assembled state into lap [ie][4][sc] (1: FP64, 2: the mixed form's FP32
+// laplacians)
+struct StateDssArgs {
+  MetricPtrs m;
+  const int *src;
+  int nelem, nlev, chunk, lap1;  // chunk: state_chunk
+  const double *pre;  // [ie][4][sc]
+  double *v, *t, *dp;
+  double *lap;
+  double nu_ratio1;
 };
 
 constexpr int DSS_MAX_FIELDS = 8;
@@ -38,61 +62,22 @@ struct DssArgs {
   int f32;               // fields hold FP32 values (accumulated in FP64)
   const int *src;        // [ie][16][3] global point ids (ie*16 + pt) or -1
   const double *rsmp;    // multiply by rspheremp if non-null
-  // lap1 (FP64 state fields v0, v1, T, dp3d in f[0..3]): also the first
-  // hyperviscosity laplacians of the assembled state, into lap_v, lap_t,
-  // lap_dp (1: FP64, 2: the mixed form's FP32 laplacians)
-  int lap1;
-  MetricPtrs m;
-  double *lap_v, *lap_t, *lap_dp;
-  double nu_ratio1;
 };
 
 struct HvArgs {
   MetricPtrs m;
   const int *src;
-  int nelem, nlev;
-  double *v, *t, *dp;                // state at np1 (in/out)
-  double *vt_a, *tt_a, *dpt_a;      // pre-exchange buffers
-  double *vt_b, *tt_b, *dpt_b;      // second buffers
+  int nelem, nlev, chunk;            // chunk: state_chunk
+  const double *v, *t, *dp;          // the subcycle's state
+  double *vo, *to, *dpo;             // the updated state (may be the same arrays)
+  double *lap, *pre;                 // first and second laplacians [ie][4][sc]
   double *dpdiss_ave, *dpdiss_bih;
   double dt, eta_ave_w, nu, nu_s, nu_p, nu_top, nu_ratio1, nu_ratio2;
   int nsub;
-  int mixed;                        // FP32 laplacians, FP32 first-laplacian buffers
-  int consthv;                      // 0: tensor form of the second laplacian
+  int mixed;                         // FP32 laplacians, FP32 first laplacians
+  int consthv;                       // 0: tensor form of the second laplacian
+  int first;                         // the accumulators start here
 };
-
-// The first laplacians of hyperviscosity at one (element, level, point) of
-// a state (t, dp, v0, v1), into the pre-exchange buffers: FP64, or (F32) the
-// mixed form's FP32 laplacians of the values less their slab reference,
-// stored as FP32.  Every lane of the slab takes part (cross-lane reads).
-template <bool F32>
-__device__ __forceinline__ void hv_first_laplacians(const MetricPtrs &m, int ie, int pt, double nu_ratio1,
-                                                    double t, double dp, double v0, double v1, double *lt,
-                                                    double *ldp, double *lv, size_t s, size_t v) {
-  if (F32) {
-    ElemLaneF e;
-    load_elemf(m, ie, pt, e);
-    DvvLaneF d;
-    load_dvvf(m.dvv, pt, d);
-    ((float *)lt)[s] = sph_laplacef(e, d, (float)(t - slab_ref(t)));
-    ((float *)ldp)[s] = sph_laplacef(e, d, (float)(dp - slab_ref(dp)));
-    float l0, l1;
-    sph_vlaplace_contraf(e, d, (float)nu_ratio1, (float)v0, (float)v1, l0, l1);
-    ((float *)lv)[v] = l0;
-    ((float *)lv)[v + 16] = l1;
-  } else {
-    ElemLane e;
-    load_elem(m, ie, pt, e);
-    DvvLane d;
-    load_dvv(m.dvv, pt, d);
-    lt[s] = sph_laplace(e, d, t);
-    ldp[s] = sph_laplace(e, d, dp);
-    double l0, l1;
-    sph_vlaplace_contra(e, d, nu_ratio1, v0, v1, l0, l1);
-    lv[v] = l0;
-    lv[v + 16] = l1;
-  }
-}
 
 // Layout of the tracer pre-exchange buffers (qdp_pre, qbih_pre, fdss_pre):
 // levels fastest in chunks of 8 levels, [ie][field][lev/8][pt][lev%8].  One
@@ -208,13 +193,11 @@ void launch_dp3d_from_ps(hipStream_t st, int nelem, int nlev, const double *hyai
 void launch_prim_step_init(hipStream_t st, int nelem, int nlev, bool zero_diss, const double *dp_n0,
                            double *eta_dot, double *vn0, double *omega, double *dpa, double *dpb, double *derived_dp);
 void launch_caar(hipStream_t st, const CaarArgs &a);
-void launch_rk_combo(hipStream_t st, int nelem, int nlev, double *v_nm1, double *t_nm1, double *dp_nm1,
-                     const double *v_n0, const double *t_n0, const double *dp_n0);
 void launch_dss(hipStream_t st, const DssArgs &a);
-// lap1_done: the first laplacians are already in vt_a, tt_a, dpt_a (formed by
-// the previous subcycle's update); lap1_next: the update forms them for the
-// next subcycle (FP64 form)
-void launch_hv_cycle(hipStream_t st, const HvArgs &a, bool lap1_done = false, bool lap1_next = false);
+void launch_state_dss(hipStream_t st, const StateDssArgs &a);
+// one subcycle, its first laplacians in a.lap; lap1_next: the update forms
+// those of the next subcycle there
+void launch_hv_cycle(hipStream_t st, const HvArgs &a, bool lap1_next);
 void launch_euler_divdp_qmm(hipStream_t st, const EulerArgs &a);
 void launch_euler_nbr_minmax(hipStream_t st, const EulerArgs &a);
 void launch_euler_advect(hipStream_t st, const EulerArgs &a, int stage);
@@ -299,6 +282,109 @@ __device__ __forceinline__ double gather_sum(const T (&r)[4], int s0, int s1, in
   return x;
 }
 
+// Layout of the dynamics' pre-exchange buffers: chunks of C consecutive levels
+// (state_chunk), [ie][field][lev/C][pt][lev%C].  A lane holds one point's chunk
+// of levels, so it moves C*8 contiguous bytes and the 16 lanes of an element
+// and chunk whole lines; a neighbour's edge point is C levels of useful bytes
+// out of the line it is read from (one level in the [lev][pt] layout).
+template <int C>
+__host__ __device__ inline size_t sc_field(int nlev) {
+  return (size_t)((nlev + C - 1) / C) * (16 * C);
+}
+
+// Orders the arithmetic: what is computed from x after pin(x) starts there,
+// and what leads to x is done by then.  The compiler would otherwise
+// interleave the levels of a lane, and spill.
+__device__ __forceinline__ void pin(double &x) { asm volatile("" : "+v"(x)::"memory"); }
+
+typedef double d2_t __attribute__((ext_vector_type(2)));
+typedef float f2_t __attribute__((ext_vector_type(2)));
+template <typename T>
+struct vec2;
+template <>
+struct vec2<double> {
+  typedef d2_t type;
+};
+template <>
+struct vec2<float> {
+  typedef f2_t type;
+};
+
+// DSS gather of a lane's chunk (levels k0 .. k0+C-1, k0 a multiple of C) from
+// fields of that layout, summed in gather_sum's order.  es: stride between
+// elements.  The first source is absent at the 4 interior points only and
+// reads the own value there (and drops it); the other two exist at corners
+// only, so their loads are masked: unmasked they would take half of the
+// gather's L1 accesses.
+template <typename T, int C>
+struct ScGather {
+  typedef typename vec2<T>::type V;
+  gptr<T> p[4];
+  int s0, s1, s2;
+  __device__ __forceinline__ ScGather(const T *f0, size_t es, int ie, int pt, int k0, const int *src) {
+    const int *s = src + ((size_t)ie * 16 + pt) * 3;
+    s0 = s[0];
+    s1 = s[1];
+    s2 = s[2];
+    const gptr<T> f = (gptr<T>)f0 + (size_t)k0 * 16;
+    p[0] = f + (size_t)ie * es + pt * C;
+    auto at = [&](int i) { return opaque_ptr(i >= 0 ? f + (size_t)(i >> 4) * es + (i & 15) * C : p[0]); };
+    p[1] = at(s0);
+    p[2] = at(s1);
+    p[3] = at(s2);
+  }
+  // the assembled values of one field, times r
+  __device__ __forceinline__ void field(size_t off, double r, double (&y)[C]) const {
+    double x[1][C];
+    sum({off}, x);
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      y[j] = x[0][j] * r;
+      pin(y[j]);
+    }
+  }
+  // the assembled values of NF fields at offsets off[f]: x[f][level]
+  template <int NF>
+  __device__ __forceinline__ void sum(const size_t (&off)[NF], double (&x)[NF][C]) const {
+    V v[NF][4][C / 2];
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < C / 2; ++j) v[f][i][j] = ((gptr<V>)(p[i] + off[f]))[j];
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int i = 2; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < C / 2; ++j) v[f][i][j] = V{0, 0};
+    if (s1 >= 0) {
+#pragma unroll
+      for (int f = 0; f < NF; ++f)
+#pragma unroll
+        for (int i = 2; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < C / 2; ++j) v[f][i][j] = ((gptr<V>)(p[i] + off[f]))[j];
+    }
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int j = 0; j < C; ++j) {
+        const T c[4] = {v[f][0][j >> 1][j & 1], v[f][1][j >> 1][j & 1], v[f][2][j >> 1][j & 1], v[f][3][j >> 1][j & 1]};
+        x[f][j] = gather_sum(c, s0, s1, s2);
+      }
+  }
+};
+
+// a lane's chunk of levels into that layout
+template <typename T, int C>
+__device__ __forceinline__ void sc_store(T *p, const T (&x)[C]) {
+  typedef typename vec2<T>::type V;
+#pragma unroll
+  for (int j = 0; j < C; j += 2) *(V *)(p + j) = V{x[j], x[j + 1]};
+}
+
 // XCD-aware block order: consecutive logical blocks stay on one XCD (one L2)
 __device__ __forceinline__ int xcd_block(int b, int n) {
   const int q = n >> 3, r = n & 7, x = b & 7;
@@ -326,6 +412,30 @@ __device__ __forceinline__ bool group_slab(int nelem, int nlev, int &ie, int &k,
   const int g = (int)(r / nelem);
   k = g * GL + kk;
   return g < (nlev + GL - 1) / GL && k < nlev;
+}
+
+// Levels per lane of the dynamics kernels.  Four, but six for 65 to 96 levels:
+// a CAAR block is one element, and blocks of five waves leave half of a CU's
+// wave slots empty (the dispatcher puts the first and fifth wave of every
+// block on the same SIMD).  CAAR at ne30, per level and step: 15.0 us at 64
+// levels (four waves), 19.2 us at 72 with four levels per lane (five waves).
+// The vertical advection of rsplit == 0 needs the registers.
+inline int state_chunk(int nlev, bool rsplit0) { return !rsplit0 && nlev > 64 && nlev <= 96 ? 6 : 4; }
+
+// Lane mapping of the other kernels on that layout: a 16-lane group is one
+// element's chunk of levels; elements first, so that neighbour copies come
+// from L2
+template <int C>
+inline int sc_blocks(int nelem, int nlev) {
+  return (int)(((long long)nelem * ((nlev + C - 1) / C) + 15) / 16);
+}
+template <int C>
+__device__ __forceinline__ bool sc_lane(int nelem, int nlev, int &ie, int &k0, int &pt) {
+  const long long s = (long long)xcd_block(blockIdx.x, gridDim.x) * 16 + (threadIdx.x >> 4);
+  pt = threadIdx.x & 15;
+  ie = (int)(s % nelem);
+  k0 = (int)(s / nelem) * C;
+  return k0 < nlev;
 }
 
 }  // namespace hx
