@@ -38,23 +38,6 @@ __device__ __forceinline__ double virtual_t(double qv, double t, double dp) {
   return t * qt;
 }
 
-// serial scan of the R rows (a multiple of 8) of one column of an LDS array x
-// (stride 16) into y, eight rows a batch: the batch's reads are one wait, and
-// nothing in it branches; f: value -> stored
-template <bool UP, typename F>
-__device__ __forceinline__ void column_scan(const double *x, double *y, int R, F f) {
-  for (int b = 0; b < R; b += 8) {
-    const int r0 = (UP ? R - 8 - b : b) * 16;
-    double r[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) r[i] = x[r0 + (UP ? 7 - i : i) * 16];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) r[i] = f(r[i]);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) y[r0 + (UP ? 7 - i : i) * 16] = r[i];
-  }
-}
-
 // LDS rows: the lanes' levels, whole batches of eight (the lanes past the last
 // level cover the rest: a wave is 4*CL levels)
 template <int CL>

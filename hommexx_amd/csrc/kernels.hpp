@@ -385,6 +385,23 @@ __device__ __forceinline__ void sc_store(T *p, const T (&x)[C]) {
   for (int j = 0; j < C; j += 2) *(V *)(p + j) = V{x[j], x[j + 1]};
 }
 
+// serial scan of the R rows (a multiple of 8) of one column of an LDS array x
+// (stride 16) into y, eight rows a batch: the batch's reads are one wait, and
+// nothing in it branches; f: value -> stored
+template <bool UP, typename F>
+__device__ __forceinline__ void column_scan(const double *x, double *y, int R, F f) {
+  for (int b = 0; b < R; b += 8) {
+    const int r0 = (UP ? R - 8 - b : b) * 16;
+    double r[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) r[i] = x[r0 + (UP ? 7 - i : i) * 16];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) r[i] = f(r[i]);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) y[r0 + (UP ? 7 - i : i) * 16] = r[i];
+  }
+}
+
 // XCD-aware block order: consecutive logical blocks stay on one XCD (one L2)
 __device__ __forceinline__ int xcd_block(int b, int n) {
   const int q = n >> 3, r = n & 7, x = b & 7;

@@ -12,6 +12,8 @@
 // that depend on the thicknesses only (the reference's ppmdx rows) and the
 // target table are evaluated once per column and shared through LDS by all
 // the fields of the element's block.
+#include <type_traits>
+
 #include "kernels.hpp"
 
 namespace hx {
@@ -95,6 +97,397 @@ __device__ __forceinline__ void ppm_parabola(double al, double ar, double a, dou
   c2 = 3.0 * (-2.0 * a + (al + ar));
 }
 
+// ------------------------------------------------------------ split columns
+// Block = element; a wave remaps one field at a time: its four 16-lane groups
+// hold the 16 columns' levels in four runs of n = ceil(nlev/4), so a field's
+// levels are loaded at once into registers (before the first output
+// overwrites them) and its sweep is nlev/4 + 4 steps long.  A group starts
+// three cells early, for the slopes, edge values and parabola that its first
+// target may need, and takes the mass of the cells above from the group above
+// (the serial sum goes round the groups, in the reference's order).
+//
+// A step finishes the parabola of cell c and then target c-1, whose lower
+// interface lies in cell c-2, c-1 or c: the three parabolas stay in registers
+// and a select takes the right one, so the 16 columns store the same level
+// together and no lane waits for another's second target.  If an interface of
+// the element moved further (an upward shift by more than a layer), the block
+// sweeps each field with one lane a column instead (remap_column).
+//
+// What depends on the column only is computed once per block and shared
+// through LDS: the grid factors of every cell (the reference's ppmdx rows), the
+// cell thicknesses and their reciprocals, and for each target level the source
+// cell kid that holds its lower interface, the offset z2 in it and the
+// reciprocal target thickness.  The thickness sums are serial scans by the
+// first 16 lanes; each (target, column) then searches by itself, from the
+// interface of its own level (the sums grow, so the reference's search, which
+// goes on from the last target's interface, ends at the same one).
+//
+// Bound: the latency of a block's chain, about 8 us of tables and 10 us a round
+// of fields (one block of 8 or 12 waves fills a CU's LDS).
+constexpr int RG2 = 10;  // grid factors, thickness and its reciprocal, per cell
+// the most levels whose tables fit the 160 KB of LDS (80 levels: 152 KB)
+constexpr int REMAP_SPLIT_NLEV = 80;
+
+__host__ __device__ inline int remap_run(int nlev) { return (nlev + 3) / 4; }
+inline size_t remap_split_lds(int nlev) {
+  const size_t lv = 4 * remap_run(nlev), rows = lv + 6;
+  const size_t sums = 2 * ((nlev + 7) & ~7) + 4;
+  return (rows * RG2 * 16 + sums * 16 + lv * (2 * 16 + 2) + 16) * 8 + lv * 16 * 2 + 16;
+}
+
+// f(0), ..., f(N-1) as straight code with constant arguments, so that register
+// arrays stay in registers
+template <int N, typename F>
+__device__ __forceinline__ void unrolled(F &&f) {
+  if constexpr (N > 0) {
+    unrolled<N - 1>(f);
+    f(std::integral_constant<int, N - 1>{});
+  }
+}
+
+// (by value: a select of array elements would put the arrays in memory)
+__device__ __forceinline__ double sel3(int i, double a, double b, double c) { return i == 0 ? a : i == 1 ? b : c; }
+
+// One field of one column, top to bottom (fac: the row of Fortran cell -2).
+// A source level is read before its target is written: cell c's parabola
+// needs levels up to c+2, and the targets found in cells up to c are at most c.
+template <typename Put>
+__device__ __forceinline__ void remap_column(const double *fac, const double *zsh, const short *ksh, int L, int alg,
+                                             const double *var, unsigned vs, bool state, Put put) {
+  auto row = [&](int j) { return fac + (j + 2) * RG2 * 16; };
+  auto mirror = [&](int r) { return r < 0 ? -r - 1 : r >= L ? 2 * L - 1 - r : r; };
+  // (mass, mean) of Fortran cell j
+  double below = 0.0;  // a(L+2) = a(L-1)
+  auto mean = [&](int j, double &m) {
+    const double *g = row(j);
+    const double x = var[(unsigned)mirror(j - 1) * vs];
+    m = state ? x * g[128] : x;
+    return div_r(m, Recip{g[128], g[144]});
+  };
+  double m0 = 0.0, m1, m2, dma0, ai_prev = 0.0, prefix = 0.0, mass_prev = 0.0;
+  double A0 = mean(0, m0), A1 = mean(1, m1), A2 = mean(2, m2), am1 = mean(-1, m0);
+  dma0 = ppm_dma_g(am1, A0, A1, row(-1)[0], row(-1)[16], row(-1)[32]);
+  int k = 0;
+  for (int j = 0; j <= L; ++j) {
+    const double *g = row(j);
+    const double dma1 = ppm_dma_g(A0, A1, A2, g[0], g[16], g[32]);
+    const double gai[5] = {g[48], g[64], g[80], g[96], g[112]};
+    const double ai = ppm_ai_g(A0, A1, dma0, dma1, gai);
+    if (j >= 1) {
+      const int c = j - 1;
+      double cc0, cc1, cc2;
+      ppm_parabola(ai_prev, ai, A0, cc0, cc1, cc2);
+      if (alg == 2 && (c <= 1 || c >= L - 2)) {
+        cc0 = A0;
+        cc1 = 0.0;
+        cc2 = 0.0;
+      }
+      for (; k < L && ksh[k * 16] == c; ++k) {
+        const double mass = prefix + integrate_parabola(cc2, cc1, cc0, -0.5, zsh[k * 16]) * g[128];
+        put(k, k > 0 ? mass - mass_prev : mass);
+        mass_prev = mass;
+      }
+      prefix += m0;
+    }
+    if (j == L - 2) below = A1;
+    A0 = A1;
+    A1 = A2;
+    m0 = m1;
+    m1 = m2;
+    if (j + 3 <= L) A2 = mean(j + 3, m2);
+    else A2 = j + 3 == L + 1 ? A1 : below;
+    dma0 = dma1;
+    ai_prev = ai;
+  }
+}
+
+template <int N, int FB>
+__global__ __launch_bounds__(FB == 1 ? 768 : 512) void remap_split_kernel(RemapArgs a) {
+  extern __shared__ double rsm[];
+  const int L = a.nlev, n = remap_run(L), nt = blockDim.x;
+  const int L4 = 4 * n;  // the groups' levels
+  // row of Fortran cell j = -2..4n+3: j+2 (past the column: the mirrored cell)
+  double *const fac = rsm;                              // [4n+6][RG2][16]
+  double *const pio = fac + (L4 + 6) * RG2 * 16;        // source interfaces 0..L+1, rows for whole batches
+  const int R = (L + 7) & ~7;
+  double *const pin = pio + (R + 2) * 16;               // target interfaces 0..L
+  double *const zsh = pin + (R + 2) * 16;               // z2 [L4][16]
+  double *const rtk = zsh + L4 * 16;                    // 1 / target thickness [L4][16]
+  double *const dab = rtk + L4 * 16;                    // hyai(k+1) - hyai(k), hybi(k+1) - hybi(k)  [L4][2]
+  double *const pss = dab + L4 * 2;                     // ps [16]
+  int *const deep = (int *)(pss + 16);                  // a target lies in none of its three cells
+  short *const ksh = (short *)(deep + 4);               // kid [L4][16]
+  double *const dxs = rtk;                              // first the source thicknesses
+  const int ie = xcd_block(blockIdx.x, gridDim.x);
+  const int tid = threadIdx.x;
+  bool bad = false;
+  {
+    const double *s0 = (a.nstates ? a.dp : a.src) + (size_t)ie * L * 16;
+    for (int i = tid; i < L * 16; i += nt) {
+      const double x = s0[i];
+      if (a.nstates) bad |= isnan(x) || x < 0.0;
+      dxs[i] = x;
+      pin[i] = x;
+    }
+    for (int i = L * 16 + tid; i < R * 16; i += nt) pin[i] = 0.0;
+    for (int k = tid; k < L; k += nt) {
+      dab[2 * k] = a.hyai[k + 1] - a.hyai[k];
+      dab[2 * k + 1] = a.hybi[k + 1] - a.hybi[k];
+    }
+    for (int i = L * 16 + tid; i < L4 * 16; i += nt) {  // (levels past the last: any cell)
+      ksh[i] = (short)(i >> 4);
+      zsh[i] = 0.0;
+    }
+    if (tid == 0) *deep = 0;
+    if (bad) atomicOr(a.error, 1);
+  }
+  __syncthreads();
+  auto target = [&](int k, double ps) { return dab[2 * k] * a.ps0 + dab[2 * k + 1] * ps; };
+  // the mirrored ghosts are dx(0) = dx(1), dx(-1) = dx(2), dx(L+1) = dx(L),
+  // dx(L+2) = dx(L-1) (cells further out only feed values nothing uses)
+  auto mirror = [&](int r) {
+    r = r < 0 ? -r - 1 : r;
+    r = r >= L ? 2 * L - 1 - r : r;
+    return r < 0 ? 0 : r;
+  };
+  if (tid < 64) {
+    // the first wave: the source interfaces, ps = sum(dp3d) + hyai0*ps0
+    // (rsplit == 0: formed with the source thicknesses), the target interfaces
+    if (tid < 16) {
+      // (the rows past the last, up to a batch of eight: zero thickness)
+      double s = 0.0;
+      pio[tid] = 0.0;
+      column_scan<false>(pin + tid, pio + 16 + tid, R, [&](double x) { return s += x; });
+      pio[(L + 1) * 16 + tid] = s + 1.0;
+      double ps;
+      if (a.nstates) {
+        ps = s + a.hyai0 * a.ps0;
+        a.ps[(size_t)ie * 16 + tid] = ps;
+      } else {
+        ps = a.ps[(size_t)ie * 16 + tid];
+      }
+      pss[tid] = ps;
+      double t = 0.0;
+      for (int b = 0; b < L; b += 8) {
+        double r[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) r[i] = target(b + i < L ? b + i : L - 1, ps);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          t += r[i];
+          pin[(b + i + 1) * 16 + tid] = t;
+        }
+      }
+      pin[L * 16 + tid] = s;
+    }
+  } else {
+    // meanwhile the others: the grid factors
+    for (int i = tid - 64; i < (L4 + 6) * 16; i += nt - 64) {
+      const int j = (i >> 4) - 2, p = i & 15;
+      // dma(j+1) factors from cells j..j+2, ai(j) factors from cells j-1..j+2
+      auto dxf = [&](int m) { return dxs[mirror(m - 1) * 16 + p]; };
+      const double Xm1 = dxf(j - 1), X0 = dxf(j), X1 = dxf(j + 1), X2 = dxf(j + 2);
+      double *g = fac + (size_t)(j + 2) * RG2 * 16 + p;
+      g[0] = X1 / (X0 + X1 + X2);
+      g[16] = (2.0 * X0 + X1) / (X1 + X2);
+      g[32] = (X1 + 2.0 * X2) / (X0 + X1);
+      g[48] = X0 / (X0 + X1);
+      g[64] = 1.0 / (Xm1 + X0 + X1 + X2);
+      g[80] = (2.0 * X0 * X1) / (X0 + X1) * ((Xm1 + X0) / (2.0 * X0 + X1) - (X2 + X1) / (2.0 * X1 + X0));
+      g[96] = X0 * (Xm1 + X0) / (2.0 * X0 + X1);
+      g[112] = X1 * (X1 + X2) / (X0 + 2.0 * X1);
+      g[128] = X0;
+      g[144] = 1.0 / X0;
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < L * 16; i += nt) {
+    const int k = i >> 4, p = i & 15;
+    const double pk = pin[(k + 1) * 16 + p];
+    int si = k;
+    while (si <= L && pio[si * 16 + p] <= pk) ++si;
+    if (si == L + 1) si = L;
+    const int kid = si - 1;
+    ksh[i] = (short)kid;
+    zsh[i] = kid >= 0 ? (pk - (pio[kid * 16 + p] + pio[si * 16 + p]) * 0.5) / fac[((kid + 3) * RG2 + 8) * 16 + p] : 0.0;
+    rtk[i] = 1.0 / target(k, pss[p]);
+    if (kid > k + 1) *deep = 1;
+    if (kid < 0) atomicOr(a.error, 2);  // below the first interface: not a column the reference remaps
+  }
+  __syncthreads();
+
+  // ------------------------------------------------------------ fields
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = nt >> 6;
+  const int lane = tid & 63, pt = lane & 15, grp = lane >> 4;
+  const int c0 = grp * n;
+  const int nf = a.nstates + a.qsize, f0 = 3 - a.nstates;  // field 0,1: v components, 2: T, >= 3: tracers
+  const double ps = pss[pt];
+  const bool general = *deep;
+  // the lane's rows of the tables: Fortran cell c0-2, target c0
+  const double *const fg = fac + c0 * RG2 * 16 + pt;
+  const double *const zg = zsh + c0 * 16 + pt, *const rg = rtk + c0 * 16 + pt, *const dg = dab + 2 * c0;
+  const short *const kg = ksh + c0 * 16 + pt;
+  // the value of the group above (garbage in group 0)
+  auto above = [&](double x) {
+    const int src = (lane - 16) * 4;
+    return mk64(__builtin_amdgcn_ds_bpermute(src, hi32(x)), __builtin_amdgcn_ds_bpermute(src, lo32(x)));
+  };
+  for (int fi = wave * FB; fi < nf; fi += nw * FB) {
+    // (a slot past the last field repeats the last one, without stores)
+    bool state[FB], on[FB];
+    unsigned vs[FB];
+    double *var[FB], *Qout[FB];
+#pragma unroll
+    for (int b = 0; b < FB; ++b) {
+      on[b] = fi + b < nf;
+      const int f = f0 + (on[b] ? fi + b : nf - 1);
+      state[b] = f < 3;
+      vs[b] = f < 2 ? 32 : 16;
+      var[b] = f < 2    ? a.v + (size_t)ie * L * 32 + f * 16
+               : f == 2 ? a.t + (size_t)ie * L * 16
+                        : a.qdp + ((size_t)ie * a.qsize + (f - 3)) * L * 16;
+      Qout[b] = f >= 3 && a.Q ? a.Q + ((size_t)ie * a.qsize + (f - 3)) * L * 16 : nullptr;
+    }
+    const unsigned qo = (unsigned)c0 * 16 + pt;
+    // target c0 + i of the lane
+    auto put = [&](int b, int i, double out, const Recip &rt) {
+      const unsigned vo = (unsigned)c0 * vs[b] + pt;
+      double *const p = var[b] + i * (int)vs[b];
+      if (state[b]) {
+        p[vo] = div_r(out, rt);
+      } else {
+        p[vo] = out;
+        if (Qout[b]) (Qout[b] + i * 16)[qo] = div_r(out, rt);
+      }
+    };
+    auto thickness = [&](int i) { return Recip{dg[2 * i] * a.ps0 + dg[2 * i + 1] * ps, rg[i * 16]}; };
+    if (general) {
+#pragma unroll
+      for (int b = 0; b < FB; ++b)
+        if (grp == 0 && on[b])
+          remap_column(fg, zg, kg, L, a.remap_alg, var[b] + pt, vs[b], state[b],
+                       [&](int i, double out) { put(b, i, out, thickness(i)); });
+      continue;
+    }
+    // levels c0-3 .. c0+n+2, all in registers before the first store
+    double v[FB][N + 6];
+#pragma unroll
+    for (int b = 0; b < FB; ++b)
+#pragma unroll
+      for (int i = 0; i < N + 6; ++i) v[b][i] = var[b][(unsigned)mirror(c0 - 3 + i) * vs[b] + pt];
+#pragma unroll
+    for (int b = 0; b < FB; ++b) {
+#pragma unroll
+      for (int i = 0; i < N + 6; ++i) hx::pin(v[b][i]);
+      if (state[b]) {
+#pragma unroll
+        for (int i = 0; i < N + 6; ++i)
+          if (i < n + 6) v[b][i] *= fg[(i * RG2 + 8) * 16];
+      }
+    }
+    // the mass above level c0-1: the sum over the levels, from each group to
+    // the next (three rounds; all groups add, one more is final in each)
+    double vtop[FB], prefix[FB] = {};  // vtop: level c0-1 as a cell (none above the column)
+#pragma unroll
+    for (int b = 0; b < FB; ++b) vtop[b] = grp ? v[b][2] : 0.0;
+#pragma unroll 1
+    for (int g = 1; g < 4; ++g) {
+      double s[FB];
+#pragma unroll
+      for (int b = 0; b < FB; ++b) s[b] = prefix[b] + vtop[b];
+#pragma unroll
+      for (int i = 3; i < N + 2; ++i)
+        if (i < n + 2)
+#pragma unroll
+          for (int b = 0; b < FB; ++b) s[b] += v[b][i];
+#pragma unroll
+      for (int b = 0; b < FB; ++b) {
+        s[b] = above(s[b]);
+        prefix[b] = grp ? s[b] : 0.0;
+      }
+    }
+    double A0[FB], A1[FB], dma0[FB] = {}, ai_prev[FB] = {}, mass[FB] = {}, mfirst[FB] = {};
+    {
+      const Recip r0{fg[8 * 16], fg[9 * 16]}, r1{fg[(RG2 + 8) * 16], fg[(RG2 + 9) * 16]};
+#pragma unroll
+      for (int b = 0; b < FB; ++b) {
+        A0[b] = div_r(v[b][0], r0);
+        A1[b] = div_r(v[b][1], r1);
+      }
+    }
+    // parabola and mass above of the last three cells
+    double q0[FB][3] = {}, q1[FB][3] = {}, q2[FB][3] = {}, qp[FB][3] = {};
+    unrolled<N + 4>([&](auto ic) __attribute__((always_inline)) {
+      constexpr int i = ic;
+      // (c and n are made anew in each step: hoisted out of the field loop, the
+      // conditions on them filled the scalar registers)
+      int nn = n, c = c0 + i - 3;  // c: the cell
+      asm volatile("" : "+s"(nn));
+      asm volatile("" : "+v"(c));
+      if (i >= nn + 4) return;
+      const double *g = fg + i * RG2 * 16;  // Fortran cell j = c0 - 2 + i
+      const double h0 = g[0], h1 = g[16], h2 = g[32];
+      const double gai[5] = {g[48], g[64], g[80], g[96], g[112]};
+      const Recip r2{g[(2 * RG2 + 8) * 16], g[(2 * RG2 + 9) * 16]};
+      constexpr int s = i % 3, s1 = (i + 2) % 3, s2 = (i + 1) % 3;  // its slot, and of cells c-1, c-2
+      int up = 0;
+      double z2 = 0.0, dx = 0.0;
+      Recip rt{};
+      if (i >= 4) {
+        up = c - kg[(i - 4) * 16];  // 0, 1 or 2 cells above, for target c-1
+        dx = g[8 * 16 - up * (RG2 * 16)];
+        z2 = zg[(i - 4) * 16];
+        rt = thickness(i - 4);
+      }
+#pragma unroll
+      for (int b = 0; b < FB; ++b) {
+        const double A2 = div_r(v[b][i + 2], r2);
+        const double dma1 = ppm_dma_g(A0[b], A1[b], A2, h0, h1, h2);         // dma(j+1)
+        const double ai = ppm_ai_g(A0[b], A1[b], dma0[b], dma1, gai);  // ai(j)
+        if (i >= 2) {
+          ppm_parabola(ai_prev[b], ai, A0[b], q0[b][s], q1[b][s], q2[b][s]);
+          if (a.remap_alg == 2 && (c <= 1 || c >= L - 2)) {
+            q0[b][s] = A0[b];
+            q1[b][s] = 0.0;
+            q2[b][s] = 0.0;
+          }
+          qp[b][s] = prefix[b];
+          if (i >= 4) {
+            const double p0 = sel3(up, q0[b][s], q0[b][s1], q0[b][s2]);
+            const double p1 = sel3(up, q1[b][s], q1[b][s1], q1[b][s2]);
+            const double p2 = sel3(up, q2[b][s], q2[b][s1], q2[b][s2]);
+            const double pp = sel3(up, qp[b][s], qp[b][s1], qp[b][s2]);
+            const double m = pp + integrate_parabola(p2, p1, p0, -0.5, z2) * dx;
+            if (i == 4) mfirst[b] = m;
+            else if (c - 1 < L && on[b]) put(b, i - 4, m - mass[b], rt);
+            mass[b] = m;
+          }
+          prefix[b] += i == 2 ? vtop[b] : v[b][i];
+        }
+        A0[b] = A1[b];
+        A1[b] = A2;
+        dma0[b] = dma1;
+        ai_prev[b] = ai;
+      }
+      // (a step's loads and arithmetic stay in it)
+#pragma unroll
+      for (int b = 0; b < FB; ++b) {
+        hx::pin(A0[b]);
+        hx::pin(A1[b]);
+        hx::pin(dma0[b]);
+        hx::pin(ai_prev[b]);
+      }
+    });
+    // a group's first target takes the mass of the last one above it
+#pragma unroll
+    for (int b = 0; b < FB; ++b) {
+      const double m = above(mass[b]);
+      if (c0 < L && on[b]) put(b, 0, grp ? mfirst[b] - m : mfirst[b], thickness(0));
+    }
+  }
+}
+
+// ---------------------------------------------------------- one lane a column
 // One block = one element (16 GLL columns) and up to 16*RFB fields; lane
 // (row, pt) sweeps column pt for fields f0 + (16*blockIdx.y + row)*RFB + i
 // (field 0,1: v components, 2: T, >= 3: tracer field-3).  What depends on
@@ -404,11 +797,44 @@ void launch_ps_from_dp(hipStream_t st, int nelem, int nlev, double hyai0, double
   hipLaunchKernelGGL(ps_from_dp_kernel, dim3((ncol + 255) / 256), dim3(256), 0, st, nelem, nlev, hyai0, ps0, dp, ps);
 }
 
+// Split columns are the shorter chain, one lane a column the fewer
+// instructions a field (its lanes share a column's tables over up to 4 fields).
+// Measured, us, split against one lane a column (with its thickness kernel):
+//   few fields:    ne30 L72 3 fields 456/812, 7 fields L26 257/291, L40 385/435
+//   long columns:  ne30 L72 15 fields 942/1137, 23 1276/1523, 27 1641/1583,
+//                  43 2319/1981; L40 15 fields 624/545, L26 15 fields 440/365
+//   few elements:  ne4 L26 7 fields 17/52, 43 51/76; ne8 L72 43 217/253, L26 43
+//                  104/102; ne11 (726 elements) L26 43 157/129
+constexpr int REMAP_SPLIT_ELEMS = 512;  // two blocks per CU
+static bool remap_split(int nelem, int nlev, int nfld) {
+  if (nlev > REMAP_SPLIT_NLEV || nfld == 0) return false;
+  return nfld <= 8 || (nlev > 64 && nfld <= 24) || nelem <= REMAP_SPLIT_ELEMS;
+}
+
 void launch_remap(hipStream_t st, const RemapArgs &a) {
-  const size_t ncol = (size_t)a.nelem * 16;
-  hipLaunchKernelGGL(remap_thickness_kernel, dim3((ncol + 255) / 256), dim3(256), 0, st, a);
   const int nfld = a.nstates + a.qsize;
+  const bool split = remap_split(a.nelem, a.nlev, nfld);
+  // (the split kernel forms ps itself; the source thicknesses of rsplit == 0
+  // need it first)
+  if (!split || !a.nstates) {
+    const size_t ncol = (size_t)a.nelem * 16;
+    hipLaunchKernelGGL(remap_thickness_kernel, dim3((ncol + 255) / 256), dim3(256), 0, st, a);
+  }
   if (nfld == 0) return;
+  if (split) {
+    const size_t lds = remap_split_lds(a.nlev);
+    const int n = remap_run(a.nlev);
+    // two fields a wave (eight waves, 256 VGPRs) where twelve waves of one
+    // would need a second round: ne60 L72 13 fields 3.35 ms against 3.55
+    const bool two = nfld > 12;
+    // (where only one block fits a CU's LDS, spare waves help with the tables)
+    const int waves = two ? 8 : lds > 80 * 1024 ? 12 : nfld < 4 ? 4 : nfld;
+    auto go = [&](auto *kernel) { hipLaunchKernelGGL(kernel, dim3(a.nelem), dim3(64 * waves), lds, st, a); };
+    if (n <= 8) go(two ? remap_split_kernel<8, 2> : remap_split_kernel<8, 1>);
+    else if (n <= 18) go(two ? remap_split_kernel<18, 2> : remap_split_kernel<18, 1>);
+    else go(two ? remap_split_kernel<20, 2> : remap_split_kernel<20, 1>);
+    return;
+  }
   // fields per lane: as few as fill the 16 rows (at most 4, then more
   // blocks per element)
   const int rfb = nfld <= 16 ? 1 : nfld <= 32 ? 2 : nfld <= 48 ? 3 : 4;
