@@ -86,8 +86,8 @@ struct Ctx {
   // scratch
   double *pre[2] = {};   // pre-exchange states [ie][4][sc] (state_chunk)
   double *cdiv = nullptr;
-  double *qdp_pre = nullptr, *qbih = nullptr, *qbih_pre = nullptr, *qlim[2] = {}, *fdss_pre = nullptr;
-  // stage-2 pre-exchange buffers: qdp_pre2 (later qbih) and an alias of
+  double *qdp_pre = nullptr, *qlim[2] = {}, *fdss_pre = nullptr;
+  // stage-2 pre-exchange buffers: qdp_pre2 and an alias of
   // pre[0], which is free during the tracer step
   double *qdp_pre2 = nullptr, *fdss_pre2 = nullptr;
   int *err_d = nullptr;
@@ -307,23 +307,19 @@ void alloc_work() {
   Ctx &c = C();
   if (c.be_set) return;
   const size_t e3 = (size_t)c.nelem * c.nlev * 16;
-  const size_t q3 = e3 * (c.qsize ? c.qsize : 1);
   // pre-exchange buffers: whole 8-level chunks per element and field
   const size_t e3c = (size_t)c.nelem * lc_field(c.nlev), q3c = e3c * (c.qsize ? c.qsize : 1);
   const size_t sc = c.nelem * std::max(sc_field<4>(c.nlev), sc_field<6>(c.nlev));
   for (double *&p : c.pre) p = dalloc<double>(std::max(4 * sc, e3c));
   c.cdiv = dalloc<double>(e3);
-  // Five 40-F3 tracer uses share two allocations (at Q = 40); no kernel
+  // Four 40-F3 tracer uses share two allocations (at Q = 40); no kernel
   // writes the allocation it gathers from:
-  //   qdp_pre : stage-1 pre-exchange (-> the stage-2 gather), then the first
-  //             laplacian of the biharmonic (the stage-2 exchange -> bih_post),
-  //             then the stage-3 pre-exchange (-> euler_dss)
-  //   qdp_pre2: stage-2 pre-exchange (-> the stage-2 exchange), then the
-  //             biharmonic result qbih (bih_post -> stage-3 advection)
+  //   qdp_pre : stage-1 pre-exchange (-> stage 2), then the first laplacian of
+  //             the biharmonic (-> stage 3)
+  //   qdp_pre2: stage-2 pre-exchange (-> its exchange), then the stage-3
+  //             pre-exchange (-> its exchange)
   c.qdp_pre = dalloc<double>(q3c);
-  c.qbih_pre = c.qdp_pre;
-  c.qdp_pre2 = dalloc<double>(q3c > q3 ? q3c : q3);
-  c.qbih = c.qdp_pre2;
+  c.qdp_pre2 = dalloc<double>(q3c);
   c.qlim[0] = dalloc<double>((size_t)c.nelem * (c.qsize ? c.qsize : 1) * ql_row(c.nlev));
   c.qlim[1] = dalloc<double>((size_t)c.nelem * (c.qsize ? c.qsize : 1) * ql_row(c.nlev));
   c.fdss_pre = dalloc<double>(e3c);
@@ -524,9 +520,6 @@ void advec_tracers(double dt) {
   a.nelem = c.nelem;
   a.nlev = c.nlev;
   a.qsize = c.qsize;
-  a.qdp_pre = c.qdp_pre;
-  a.qbih = c.qbih;
-  a.qbih_pre = c.qbih_pre;
   a.derived_dp = c.derived_dp;
   a.divdp = c.divdp;
   a.divdp_proj = c.divdp_proj;
@@ -564,68 +557,52 @@ void advec_tracers(double dt) {
     a.qlim = c.qlim[cur];
   };
   nbr_minmax();
-  bool qmm_done = false;  // stage-3 bounds and first laplacian formed by the stage-2 exchange
-  for (int stage = 0; stage < 3; ++stage) {
-    const int n0q = stage == 0 ? c.n0_qdp : c.np1_qdp;
-    a.qdp_n0 = c.qdp[n0q];
-    a.qdp_np1 = c.qdp[c.np1_qdp];
-    a.rhs_multiplier = (double)stage;
-    a.rhs_viss = stage == 2 ? 3.0 : 0.0;
-    a.fdss = stage == 0 ? c.divdp_proj : stage == 1 ? c.eta_dot : c.omega;
-    // (stage 3 reads qbih from the other allocation)
-    a.qdp_pre = c.qdp_pre;
-    a.qdp_avg_n0 = stage == 2 ? c.qdp[c.n0_qdp] : nullptr;
-    // stage 2 gathers stage 1's exchange itself (the assembled stage-1 Qdp
-    // is never stored) unless the caller stops after stage 1
-    const bool fuse1 = c.debug_stop != 4;
-    if (stage == 1 && fuse1) {
-      EulerArgs b = a;
-      b.qdp_pre_in = c.qdp_pre;
-      b.fdss_pre_in = c.fdss_pre;
-      b.qdp_pre = c.qdp_pre2;
-      b.fdss_pre = c.fdss_pre2;
-      {
-        Scope s("euler_advect");
-        launch_euler_advect_gather(c.st, b);
-      }
-      b.fdss = c.eta_dot;
-      // the exchange also forms the stage-3 bounds and the first laplacian
-      // of the biharmonic (the qmm_lap step below) when the form allows
-      b.rhs_multiplier = 2.0;
-      Scope s("euler_dss_qmm");
-      qmm_done = launch_euler_dss_qmm(c.st, b);
-      if (!qmm_done) {
-        b.rhs_multiplier = 1.0;
-        launch_euler_dss(c.st, b, 0);
-      }
-    } else {
-      {
-        Scope s("euler_advect");
-        launch_euler_advect(c.st, a, stage + 1);
-      }
-      if (!(stage == 0 && fuse1)) {
-        Scope s("euler_dss");
-        launch_euler_dss(c.st, a, stage == 2);
-      }
-    }
-    if (stage == 0 && stop_here(4)) return;
-    if (stage == 1) {
-      // stage-3 bounds and tracer biharmonic from the assembled stage-2 Qdp
-      EulerArgs b = a;
-      b.qdp_n0 = c.qdp[c.np1_qdp];
-      b.rhs_multiplier = 2.0;
-      b.rhs_viss = 3.0;
-      if (!qmm_done) {
-        Scope s("euler_qmm_lap");
-        launch_euler_qmm_lap(c.st, b);
-      }
-      {
-        Scope s("euler_bih_post");
-        launch_euler_bih_post(c.st, b);
-      }
-      nbr_minmax();
-    }
+  const double *qdp_n0 = c.qdp[c.n0_qdp];
+  double *qdp_np1 = c.qdp[c.np1_qdp];
+  a.qdp_np1 = qdp_np1;
+  // stage 1: Qdp(n0) -> qdp_pre
+  a.qdp_n0 = qdp_n0;
+  a.fdss = c.divdp_proj;
+  a.qdp_pre = c.qdp_pre;
+  a.fdss_pre = c.fdss_pre;
+  {
+    Scope s("euler_advect");
+    launch_euler_advect(c.st, a, 1);
   }
+  if (c.debug_stop == 4) {
+    launch_euler_dss(c.st, a, 0);
+    stop_here(4);
+    return;
+  }
+  // stage 2: gathers qdp_pre, -> qdp_pre2
+  a.qdp_pre_in = c.qdp_pre;
+  a.fdss_pre_in = c.fdss_pre;
+  a.fdss = c.eta_dot;
+  a.qdp_pre = c.qdp_pre2;
+  a.fdss_pre = c.fdss_pre2;
+  {
+    Scope s("euler_advect");
+    launch_euler_advect(c.st, a, 2);
+  }
+  // its exchange: gathers qdp_pre2, -> Qdp(np1), laplacian -> qdp_pre
+  a.qbih_pre = c.qdp_pre;
+  {
+    Scope s("euler_dss_lap");
+    launch_euler_dss_lap(c.st, a);
+  }
+  nbr_minmax();
+  // stage 3: Qdp(np1), gathers qdp_pre, -> qdp_pre2, and its exchange
+  a.qdp_n0 = qdp_np1;
+  a.fdss = c.omega;
+  a.fdss_pre = c.fdss_pre;
+  a.rhs_viss = 3.0;
+  {
+    Scope s("euler_advect");
+    launch_euler_advect(c.st, a, 3);
+  }
+  a.qdp_avg_n0 = qdp_n0;
+  Scope s("euler_dss");
+  launch_euler_dss(c.st, a, 1);
 }
 
 void prim_step(double dt) {

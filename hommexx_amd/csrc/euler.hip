@@ -1,20 +1,18 @@
 // Euler tracer step with quasi-monotone limiters (EulerStepFunctorImpl.hpp
 // and prim_advec_tracers_remap.cpp in the reference).
 //
-// Slab kernels (16 lanes = one element at one level) loop over all tracers
-// of a slab, so metric, dp and vstar are loaded once per slab.  The exchange
-// kernels (DSS, biharmonic second half) are gathers and walk one field at a
-// time in level groups (group_slab) so neighbour copies come from L2.  One
-// remap interval's tracer step is
+// Every kernel loops over all tracers of its points, so metric, dp and vstar
+// are loaded once.  One remap interval's tracer step is
 //   divdp_qmm  : divdp = div(vn0); stage-1 qmin/qmax
 //   nbr_minmax
-//   advect(1)  ; dss           (extra field divdp_proj)
-//   advect(2)  (stage-2 qmin/qmax update fused: no exchange at this stage)
-//   dss        (extra field eta_dot_dpdn)
-//   qmm_lap    : stage-3 qmin/qmax and the first laplacian of the biharmonic
-//   bih_post   : DSS of the first laplacian, second laplacian, scaling
+//   advect(1)
+//   advect(2)  : gathers stage 1's exchange (extra field divdp_proj) and updates
+//                qmin/qmax
+//   dss_lap    : stage 2's exchange (extra field eta_dot_dpdn), stage-3
+//                qmin/qmax, the first laplacian of the biharmonic
 //   nbr_minmax
-//   advect(3)  ; dss + SSP average (extra field omega_p)
+//   advect(3)  : gathers the laplacian's exchange, second laplacian
+//   dss        : stage 3's exchange + SSP average (extra field omega_p)
 // Limiter sums run over the 16 points in index order (slab_sum_serial) to
 // round like the reference's serial reductions.
 #include <type_traits>
@@ -120,51 +118,144 @@ __global__ __launch_bounds__(256) void euler_nbr_minmax_kernel(EulerArgs a) {
   *(double2 *)(a.qlim_new + own) = make_double2(mn, mx);
 }
 
-// gather of point (ie, pt) at level k from pre-exchange fields (layout
-// lc_index) with element stride es: the own copy and the three sources'
-// copies (an absent source points at the own copy), in the reference's
-// order.  The four addresses are formed once per lane; field f of a batch is
-// then one offset (f * field size, uniform) added to each.  load issues the
-// four loads, gather_sum adds them (FP32 buffers of the mixed form are
-// accumulated in FP64 the same way).
+// ------------------------------------------------------------- lane mapping
+// Advection, exchanges and laplacians: a wave is one element's 8-level chunk of
+// the pre-exchange layout (lc_index), a lane one point at two levels k0, k0+1
+// of it, for every tracer.  A wave then moves whole lines in 16-byte pieces,
+// gathers its own points (no hand-off between lanes, no barrier), and two
+// levels' chains run side by side.  Elements first, then chunks: the waves
+// that run together on an XCD are neighbours at the same tracer, so neighbour
+// copies come from its L2.
+//
+// What bounds them is HBM, if enough waves are in flight: a lane's two FP64
+// chains take 100-130 registers, and the times follow the waves per SIMD which
+// that leaves.  So the code is ordered to stay at four: bounds are loaded at the
+// top of the tracer that uses them, the next tracer's gather once the
+// laplacian's registers are free, and pin() keeps the two levels' chains apart.
+// At 5400 elements, 72 levels, 40 tracers in FP64, ms:
+//                one lane a level, an exchange of its own per stage  |  now
+//   advect(1)                                        1.03            |  0.98
+//   advect(2)    1.73 with its gather, 1.23 its exchange             |  1.26
+//   dss_lap      0.96 bounds and laplacian                           |  1.57
+//   advect(3)    1.43, 1.41 second laplacian and exchange            |  1.81
+//   dss                                              1.23            |  1.19
+//   in all                                           9.02            |  6.81
+// dss, dss_lap and advect(3) move three tracer sets each (6.0 GB: 1.27 ms at the
+// copy rate); FP64 arithmetic keeps advect(3) busy for 1.25 ms besides.  Capping
+// registers with waves_per_eu spills (advect(3) 6.9 ms); two tracers' gathers
+// ahead cost a wave (advect(3) 3.1, dss_lap 2.0 ms).
+struct TLane {
+  int ie, k0, pt;
+  bool ok[2];  // the levels exist
+  int lv[2];   // level, or the last one
+};
+
+__device__ __forceinline__ bool tracer_lane(int nelem, int nlev, TLane &t) {
+  const long long w = (long long)xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6);
+  const int c = (int)(w / nelem);
+  t.ie = __builtin_amdgcn_readfirstlane((int)(w % nelem));
+  if (c * 8 >= nlev) return false;  // whole wave
+  t.pt = threadIdx.x & 15;
+  t.k0 = c * 8 + ((threadIdx.x >> 4) & 3) * 2;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    t.ok[j] = t.k0 + j < nlev;
+    t.lv[j] = t.ok[j] ? t.k0 + j : nlev - 1;
+  }
+  return true;
+}
+static int tracer_blocks(const EulerArgs &a) {
+  return (int)(((long long)a.nelem * ((a.nlev + 7) / 8) + 3) / 4);
+}
+// Small grids also split the tracers over blockIdx.y, up to TRACER_WAVES waves
+// (two per SIMD): a wave's time is its chain of tracers there, and the setup
+// that every share repeats (a fifth of a tracer's arithmetic, and loads that hit
+// L2) runs on idle units.  96 elements, 26 levels, 4 tracers (384 waves):
+// advect(3) 21.4 -> 12.0 us, advect(1) 17.9 -> 10.8, advect(2) 11.4 -> 7.5,
+// dss_lap 9.2 -> 6.3.  Above it the repeated setup costs more: 3456 waves of 4
+// tracers 23.3 -> 25.8 us for advect(3), 2904 of 7 tracers 20.3 -> 23.0 for
+// dss_lap, in two shares.
+constexpr long long TRACER_WAVES = 2048;
+static dim3 tracer_grid(const EulerArgs &a) {
+  const long long b = tracer_blocks(a);
+  long long n = (TRACER_WAVES / 4 + b - 1) / b;
+  n = n < a.qsize ? n : a.qsize;
+  return dim3((unsigned)b, (unsigned)(n > 1 ? n : 1));
+}
+// this block's share [qa, qb) of the tracers
+__device__ __forceinline__ bool tracer_share(int Q, int &qa, int &qb) {
+  const int per = (Q + gridDim.y - 1) / gridDim.y;
+  qa = blockIdx.y * per;
+  qb = qa + per < Q ? qa + per : Q;
+  return qa < qb;
+}
+
+// DSS gather of a lane's two levels from fields in the lc_index layout (element
+// stride es).  load issues the loads of the field at offset off, masked to the
+// lanes that have the source (the others read 0, which leaves a sum as it
+// is), sum adds them in the reference's order.
 template <typename T>
-struct LfGather {
+struct TGather {
+  typedef typename vec2<T>::type V;
   gptr<T> p[4];
-  __device__ __forceinline__ LfGather(const T *fg, size_t es, int ie, int pt, int k, int s0, int s1, int s2) {
-    const gptr<T> f = (gptr<T>)fg;
-    p[0] = f + (size_t)ie * es + lc_index(pt, k);
-    // (opaque: the selected address stays one unconditional load)
-    auto at = [&](int s) { return opaque_ptr(s >= 0 ? f + (size_t)(s >> 4) * es + lc_index(s & 15, k) : p[0]); };
+  bool edge, corner, third;
+  V r[4];
+  __device__ __forceinline__ TGather(const T *f0, size_t es, const TLane &t, const int *src) {
+    const int *s = src + ((size_t)t.ie * 16 + t.pt) * 3;
+    const int s0 = s[0], s1 = s[1], s2 = s[2];
+    edge = s0 >= 0;
+    corner = s1 >= 0;
+    const gptr<T> f = (gptr<T>)f0 + lc_index(0, t.k0);
+    p[0] = f + (size_t)t.ie * es + t.pt * 8;
+    auto at = [&](int i) { return i >= 0 ? f + (size_t)(i >> 4) * es + (i & 15) * 8 : p[0]; };
     p[1] = at(s0);
     p[2] = at(s1);
     p[3] = at(s2);
+    third = s2 >= 0;
   }
-  __device__ __forceinline__ void load(size_t off, T (&r)[4]) const {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) r[j] = p[j][off];
+  __device__ __forceinline__ void load(size_t off) {
+    r[0] = *(gptr<V>)(p[0] + off);
+    r[1] = r[2] = r[3] = V{0, 0};
+    if (edge) r[1] = *(gptr<V>)(p[1] + off);
+    if (corner) {
+      r[2] = *(gptr<V>)(p[2] + off);
+      if (third) r[3] = *(gptr<V>)(p[3] + off);
+    }
   }
-  __device__ __forceinline__ double sum(size_t off, int s0, int s1, int s2) const {
-    T r[4];
-    load(off, r);
-    return gather_sum(r, s0, s1, s2);
+  __device__ __forceinline__ double sum(int j) const {
+    return (((double)r[0][j] + (double)r[1][j]) + (double)r[2][j]) + (double)r[3][j];
   }
 };
 
-// The same gather with the addresses formed per field: fewer live registers
-// than LfGather's four pointers (euler_dss keeps 8 waves per SIMD with it).
-template <typename T>
-__device__ __forceinline__ double gather_lf(const T *f, size_t es, size_t off, int ie, int pt, int k, int s0, int s1,
-                                            int s2) {
-  const size_t own = (size_t)ie * es + off + lc_index(pt, k);
-  auto at = [&](int s) { return opaque_index(s >= 0 ? (size_t)(s >> 4) * es + off + lc_index(s & 15, k) : own); };
-  const T r[4] = {f[own], f[at(s0)], f[at(s1)], f[at(s2)]};
-  return gather_sum(r, s0, s1, s2);
-}
+// The weak divergence's columns of Dvv (TJ, TI) in LDS, a copy per wave: the
+// laplacians read them for each tracer instead of holding 16 registers.
+template <bool ON>
+struct WkLds {
+  d2_t *p;
+  __device__ __forceinline__ WkLds() {
+    __shared__ d2_t wk[ON ? 4 : 1][4][ON ? 64 : 1];
+    p = &wk[ON ? threadIdx.x >> 6 : 0][0][ON ? threadIdx.x & 63 : 0];
+  }
+  __device__ __forceinline__ void put(const DvvLane &d) {
+    p[0] = d2_t{d.TJ[0], d.TJ[1]};
+    p[64] = d2_t{d.TJ[2], d.TJ[3]};
+    p[128] = d2_t{d.TI[0], d.TI[1]};
+    p[192] = d2_t{d.TI[2], d.TI[3]};
+  }
+  __device__ __forceinline__ void get(DvvLane &w) const {
+    unsigned o = 0;
+    asm volatile("" : "+v"(o));  // (read here: not hoisted out of the tracer loop)
+    const d2_t w0 = p[o], w1 = p[o + 64], w2 = p[o + 128], w3 = p[o + 192];
+    w.TJ[0] = w0[0], w.TJ[1] = w0[1], w.TJ[2] = w1[0], w.TJ[3] = w1[1];
+    w.TI[0] = w2[0], w.TI[1] = w2[1], w.TI[2] = w3[0], w.TI[3] = w3[1];
+  }
+};
 
 // ------------------------------------------------------------ limiters
 // limiter_optim_iter_full (:767-823), one slab = one level of one tracer
 __device__ __forceinline__ void limit8_slab(double mass, double minp, double maxp, double &x, double c) {
   const double tol_limiter = 5e-14;
+// ( times for two levels: 40 KB of code)
   for (int iter = 0; iter < NP2 - 1; ++iter) {
     double delta = 0;
     if (x > maxp) {
@@ -217,483 +308,317 @@ __device__ __forceinline__ void limit9_slab(double minp, double maxp, double &x,
   }
 }
 
-// Setup phase (:585-626) + tracer phase (:571-687) for every tracer of an
-// (element, level) slab.  At stage 2 the qmin/qmax update of that stage
-// (min/max with the previous bounds, no neighbour exchange) runs first.
-//
-// GATHER (stage 2 only): the stage-1 exchange is done here instead of by a
-// separate kernel.  A block is one element x AGL levels (16*AGL lanes); lanes
-// (pt, kk) gather the stage-1 pre-exchange values (levels fastest) of point
-// pt at level k0+kk with the reference's accumulation order, an LDS tile
-// hands them to the slab lanes (kk, pt), and the assembled stage-1 Qdp is
-// used directly (never stored).  The assembled extra field (divdp_proj) is
-// stored, later stages read it.
-constexpr int AGL = 8;
+// the bounds of a lane's two levels (equal in the lanes of a group), by the
+// first two lanes of the group: one store of a whole line per wave
+__device__ __forceinline__ void put_bounds(double *ql, const TLane &t, d2_t b0, d2_t b1) {
+  if (t.pt < 2 && (t.pt ? t.ok[1] : t.ok[0])) *(d2_t *)(ql + 2 * t.pt) = t.pt ? b1 : b0;
+}
 
-// (at most 96 VGPRs: five waves per SIMD)
-template <bool MIXED, bool GATHER>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void euler_advect_kernel(EulerArgs a,
-                                                                                                     int stage) {
-  __shared__ double tile[GATHER ? 2 : 1][AGL][17];
-  size_t slab;
-  int ie, k, pt;
-  const int L = a.nlev, Q = a.qsize;
-  // gather role (GATHER only)
-  int gpt = 0, gk = 0, gkk = 0, kk = 0, g0 = -1, g1 = -1, g2 = -1;
-  bool gon = false, son = true;
-  double gr = 0.0;
-  if (GATHER) {
-    const int lb = xcd_block(blockIdx.x, gridDim.x);
-    ie = lb % a.nelem;
-    const int k0 = (lb / a.nelem) * AGL;
-    if (k0 >= L) return;  // whole block
-    kk = threadIdx.x >> 4;
-    pt = threadIdx.x & 15;
-    k = k0 + kk;
-    son = k < L;
-    gpt = threadIdx.x / AGL;
-    gkk = threadIdx.x % AGL;
-    gk = k0 + gkk;
-    gon = gk < L;
-    const int *src = a.src + ((size_t)ie * 16 + gpt) * 3;
-    g0 = src[0];
-    g1 = src[1];
-    g2 = src[2];
-    gr = a.m.rspheremp[(size_t)ie * 16 + gpt];
-    slab = (size_t)ie * L + (son ? k : 0);
-  } else {
-    if (!slab_ie_k((size_t)a.nelem * a.nlev, a.nlev, slab, ie, k, pt)) return;
-  }
+// The assembled extra field of a lane's levels from its pre-exchange values
+__device__ __forceinline__ void gather_extra(const EulerArgs &a, const double *pre, const TLane &t, double r,
+                                             double (&x)[2]) {
+  TGather<double> g(pre, lc_field(a.nlev), t, a.src);
+  g.load(0);
+#pragma unroll
+  for (int j = 0; j < 2; ++j) x[j] = g.sum(j) * r;
+}
+
+// Setup phase (:585-626) + tracer phase (:571-687) for every tracer: div(vstar
+// Qdp), the limiter, and the pre-exchange values of the stage.
+// Stage 1 reads Qdp(n0).  Stage 2 gathers stage 1's exchange itself (the
+// assembled stage-1 Qdp is never stored), and first updates the bounds with
+// it (no neighbour exchange at this stage).  Stage 3 reads Qdp(np1) and
+// gathers the exchange of the biharmonic's first laplacian; the second
+// laplacian (:216-310) goes straight into the update.
+// BIH: the biharmonic is 0 FP64, 1 the tensor form (FP64), 2 FP32 (mixed form).
+template <bool MIXED, int STAGE, int BIH>
+__global__ __launch_bounds__(256) void euler_advect_kernel(EulerArgs a) {
+  TLane t;
+  if (!tracer_lane(a.nelem, a.nlev, t)) return;
+  const int L = a.nlev, Q = a.qsize, pt = t.pt;
+  const size_t fs = lc_field(L), es = (size_t)Q * fs;
+  // the tracer pre-exchange values are stored in FP32 in the mixed form (the
+  // exchange sums them in FP64)
+  using PreT = typename std::conditional<MIXED, float, double>::type;
+  using LapT = typename std::conditional<BIH == 2, float, double>::type;
+  using InT = typename std::conditional<STAGE == 3, LapT, PreT>::type;
   ElemLane e;
-  load_elem_light(a.m, ie, pt, e);
+  load_elem_light(a.m, t.ie, pt, e);
   DvvLane d;
   load_dvv(a.m.dvv, pt, d);
-  const size_t s = slab * 16 + pt, v = slab * 32 + pt;
-  const double rhsmdt = a.rhs_multiplier * a.dt;
-  double dpproj;
-  const int gkc = gon ? gk : L - 1;  // gathers of a padding lane stay in bounds
-  if (GATHER) {
-    // assembled divdp_proj of stage 1
-    const double y = LfGather<double>(a.fdss_pre_in, lc_field(L), ie, gpt, gkc, g0, g1, g2).sum(0, g0, g1, g2) * gr;
-    if (gon) tile[0][gkk][gpt] = y;
-    lds_barrier();
-    dpproj = tile[0][kk][pt];
-    if (son) a.divdp_proj_w[s] = dpproj;
-    lds_barrier();
-  } else {
-    dpproj = a.divdp_proj[s];
-  }
-  const double dp = a.derived_dp[s] - rhsmdt * dpproj;
-  const double vs0 = a.vn0[v] / dp, vs1 = a.vn0[v + 16] / dp;
-  double dpdissk = dp - a.dt * a.divdp[s];
-  // (the gathering kernel runs stage 2 only, where rhs_viss == 0: no
-  // biharmonic terms, and no conditional loads that would wait for the gathers)
-  const bool add_ps_diss = !GATHER && a.nu_p > 0 && a.rhs_viss != 0.0;
-  if (add_ps_diss) {
-    const double diss_fac = -a.rhs_viss * a.dt * a.nu_q;
-    dpdissk += diss_fac * a.dpdiss_bih[s] / e.sph;
-  }
-  if (son) a.fdss_pre[(size_t)ie * lc_field(L) + lc_index(pt, k)] = a.fdss[s] * e.sph;
-  const bool add_hv = !GATHER && a.rhs_viss != 0.0;
+  const double rhsmdt = (STAGE - 1) * a.dt;
+  double dpproj[2], vs0[2], vs1[2], s1[2], fb[2];
+  Recip rdp[2], rdpd[2];
+  if (STAGE == 2) gather_extra(a, a.fdss_pre_in, t, e.rsmp, dpproj);
   const bool limit = a.limiter_option == 8 || a.limiter_option == 9;
+  double fx[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const size_t s = ((size_t)t.ie * L + t.lv[j]) * 16 + pt, v = ((size_t)t.ie * L + t.lv[j]) * 32 + pt;
+    if (STAGE == 2) {
+      if (t.ok[j] && blockIdx.y == 0) a.divdp_proj_w[s] = dpproj[j];
+    } else {
+      dpproj[j] = a.divdp_proj[s];
+    }
+    const double dp = a.derived_dp[s] - rhsmdt * dpproj[j];
+    vs0[j] = a.vn0[v] / dp;
+    vs1[j] = a.vn0[v + 16] / dp;
+    double dpdissk = dp - a.dt * a.divdp[s];
+    if (STAGE == 3 && a.nu_p > 0) {
+      const double diss_fac = -a.rhs_viss * a.dt * a.nu_q;
+      dpdissk += diss_fac * a.dpdiss_bih[s] / e.sph;
+    }
+    fx[j] = a.fdss[s] * e.sph;
+    // the divisors shared by the tracers: Qdp / dp (stage 2), ptens / dpdissk
+    if (STAGE == 2) rdp[j] = recip(dp);
+    rdpd[j] = recip(dpdissk);
+    s1[j] = limit ? slab_sum_serial(e.sph * dpdissk) : 0.0;  // same for every tracer
+    if (STAGE == 3) fb[j] = -a.rhs_viss * a.dt * a.nu_q * a.dp0[t.lv[j]];
+  }
+  if (blockIdx.y == 0) *(d2_t *)(a.fdss_pre + (size_t)t.ie * fs + lc_index(pt, t.k0)) = d2_t{fx[0], fx[1]};
+  int qa, qb;
+  if (!tracer_share(Q, qa, qb)) return;
   DvvLaneF df;
   float rmd = 0.f;
   if (MIXED) {
     load_dvvf(a.m.dvv, pt, df);
     rmd = (float)(1.0 / e.metdet * RREARTH);
   }
-  const double c = e.sph * dpdissk;
-  // the divisors shared by the tracers: Qdp / dp (stage 2), ptens / dpdissk
-  const Recip rdp = recip(dp), rdpd = recip(dpdissk);
-  const double s1 = limit ? slab_sum_serial(c) : 0.0;  // same for every tracer
-  const size_t fs = lc_field(L), es = (size_t)Q * fs;
-  // the tracer pre-exchange values are stored in FP32 in the mixed form (the
-  // exchange sums them in FP64)
-  using PreT = typename std::conditional<MIXED, float, double>::type;
-  const PreT *qpin = (const PreT *)a.qdp_pre_in;
-  PreT *qpout = (PreT *)a.qdp_pre;
-  PreT graw[4] = {};  // the loads of the next tracer's gather
-  const LfGather<PreT> gq(qpin, es, ie, gpt, gkc, g0, g1, g2);
-  if (GATHER && Q > 0) gq.load(0, graw);
-  const int kc = son ? k : L - 1;  // reads of a padding slab stay in bounds
-  // Slab path (stages 1 and 3): tracer q+1's Qdp, biharmonic term and
-  // bounds are loaded during tracer q's arithmetic.  The loads are
-  // unconditional (past the last tracer the last is reloaded; without a
-  // biharmonic term of a type, Qdp, or one FP32 value, is loaded in its
-  // place): a conditional load would make the waits that follow cover the
-  // prefetch.
-  constexpr bool PF = !GATHER;
-  const bool bihf = add_hv && a.bih32;  // FP32 biharmonic term (mixed form)
-  const double *qbp = add_hv && !a.bih32 ? a.qbih : a.qdp_n0;
-  const float *qbf = (const float *)(bihf ? a.qbih : a.qdp_n0);
-  double pf[5] = {};  // Qdp, biharmonic term (FP64, FP32), qmin, qmax of the next tracer
-  // the lane's addresses for tracer 0; tracer q adds q times a (uniform)
-  // tracer stride
-  const size_t qs = (size_t)L * 16, q0i = ((size_t)ie * Q * L + kc) * 16 + pt;
-  const double *qdp_l = a.qdp_n0 + q0i, *qbp_l = qbp + q0i;
-  const float *qbf_l = bihf ? qbf + q0i : qbf;
-  double *ql_l = a.qlim + (size_t)ie * Q * ql_row(L) + ql_min(kc);
-  PreT *qpo_l = qpout + (size_t)ie * es + lc_index(pt, kc);
+  ElemLaneF ef;
+  if (STAGE == 3 && BIH == 2) load_elemf(a.m, t.ie, pt, ef);
+  double tv[4], tvs[6];
+  if (STAGE == 3 && BIH == 1) load_tensor(a.m, t.ie, pt, tv, tvs);
+  const Recip rsph = recip(e.sph);
+  constexpr bool TLDS = STAGE == 3 && BIH != 2;
+  WkLds<TLDS> wk;
+  if (TLDS) wk.put(d);
+  // the element's parts of the arrays and the lane's offsets in them; tracer q
+  // adds q uniform strides
+  const size_t qs = (size_t)L * 16;
+  const double *const qdpE = a.qdp_n0 + (size_t)t.ie * Q * qs;
+  double *const qlE = a.qlim + (size_t)t.ie * Q * ql_row(L);
+  PreT *const outE = (PreT *)a.qdp_pre + (size_t)t.ie * es;
+  const unsigned qo0 = t.lv[0] * 16 + pt, qo1 = t.lv[1] * 16 + pt, lo = (unsigned)ql_min(t.k0),
+                 oo = (unsigned)lc_index(pt, t.k0);
+  TGather<InT> g((const InT *)(STAGE == 3 ? a.qbih_pre : a.qdp_pre_in), es, t, a.src);
+  // tracer q+1's gather (stage 1: its Qdp) is loaded during tracer q's
+  // arithmetic (past the last tracer the last is loaded again: the loads stay
+  // unconditional)
+  double nq0 = 0.0, nq1 = 0.0;
   auto fetch = [&](int q) {
-    const size_t qq = q < Q ? q : Q - 1;
-    const double2 b = *(const double2 *)(ql_l + qq * ql_row(L));
-    pf[2] = b.x;
-    pf[3] = b.y;
-    pf[0] = qdp_l[qq * qs];
-    pf[1] = qbp_l[qq * qs];
-    if (MIXED) pf[4] = qbf_l[bihf ? qq * qs : 0];
+    const size_t qq = q < qb ? q : qb - 1;
+    if (STAGE == 1) {
+      nq0 = (qdpE + qq * qs)[qo0];
+      nq1 = (qdpE + qq * qs)[qo1];
+    }
+    if (STAGE != 1) g.load(qq * fs);
   };
-  if (PF && Q > 0) fetch(0);
-  // tracer q's work; at stage 2 gcur holds tracer q's gathered loads and
-  // takes tracer q+GD's.  The mixed form (FP32 gathers, 96 VGPRs) keeps two
-  // tracers of gathers in flight (1581 against 1664 us); FP64 one (two need
-  // 112 VGPRs, 4 waves per SIMD: 1820 against 1708 us).
-  constexpr int GD = MIXED ? 2 : 1;
-  auto tracer = [&](int q, PreT (&gcur)[4]) {
-    const size_t qi = (size_t)q * qs;  // tracer q's offset from qdp_l, qbp_l, qbf_l
-    double *ql = ql_l + (size_t)q * ql_row(L);
-    double minp, maxp, qd, q0pf = 0.0;
-    if (PF) {
-      qd = pf[0];
-      q0pf = add_hv ? (bihf ? pf[4] : pf[1]) : 0.0;
-      minp = pf[2];
-      maxp = pf[3];
-      fetch(q + 1);
-    } else {
-      // this tracer's bounds are loaded before the next tracer's gather is
-      // issued: loads complete in issue order, so waiting for them does not
-      // wait for the gather
-      minp = ql[0];
-      maxp = ql[QL_MAX];
+  fetch(qa);
+  for (int q = qa; q < qb; ++q) {
+    double *const ql = qlE + (size_t)q * ql_row(L) + lo;
+    const d2_t b0 = *(const d2_t *)ql, b1 = *(const d2_t *)(ql + 2);
+    double minp[2] = {b0[0], b1[0]}, maxp[2] = {b0[1], b1[1]}, qd[2] = {nq0, nq1}, y[2];
+    if (STAGE == 3) {
+      qd[0] = (qdpE + q * qs)[qo0];
+      qd[1] = (qdpE + q * qs)[qo1];
     }
-    if (GATHER) {
-      // the stage-1 exchange of tracer q; tracer q+GD's loads are issued
-      // before this tracer's arithmetic and stay in flight across the
-      // (LDS-only) barrier
-      const double y = gather_sum(gcur, g0, g1, g2) * gr;
-      if (gon) tile[q & 1][gkk][gpt] = y;
-      // (unconditional, the last tracer reloads itself: a branch here would
-      // make every later wait cover the gathers)
-      gq.load((size_t)(q + GD < Q ? q + GD : Q - 1) * fs, gcur);
-      lds_barrier();
-      qd = tile[q & 1][kk][pt];
-    } else if (!PF) {
-      qd = qdp_l[qi];
+    if (STAGE != 1) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) y[j] = g.sum(j) * e.rsmp;
     }
-    if (stage == 2) {  // compute_qmin_qmax with rhs_multiplier == 1
-      const double xq = div_r(qd, rdp);
-      minp = dmin(minp, slab_min(xq));
-      maxp = dmax(maxp, slab_max(xq));
-    }
-    double ptens;
-    if (MIXED) {
-      // flux divergence in FP32 with compensated contractions; the update
-      // qdp - dt*div + qbih stays FP64
-      const double q0 = PF ? q0pf : (add_hv ? (bihf ? (double)qbf_l[qi] : qbp_l[qi]) : 0);
-      const double fa = vs0 * qd, fb = vs1 * qd;
-      const float gv0 = (float)((e.Dinv[0] * fa + e.Dinv[2] * fb) * e.metdet);
-      const float gv1 = (float)((e.Dinv[1] * fa + e.Dinv[3] * fb) * e.metdet);
-      const float dv = (row_contractf(df.J, gv0) + col_contractf(df.I, gv1)) * rmd;
-      ptens = (qd + -a.dt * (double)dv + q0);
-    } else {
-      ptens = sph_div_update(e, d, -a.dt, vs0, vs1, qd, q0pf);
-    }
-    bool wmin = stage == 2, wmax = stage == 2;
-    if (limit) {
-      double x = div_r(ptens, rdpd);
-      const double s0 = slab_sum_serial(x * c);
-      if (!(s1 <= 0)) {
-        if (minp < 0) {
-          minp = 0;
-          wmin = true;
-        }
-        if (s0 < minp * s1) {
-          minp = s0 / s1;
-          wmin = true;
-        }
-        if (s0 > maxp * s1) {
-          maxp = s0 / s1;
-          wmax = true;
-        }
-        if (a.limiter_option == 8) limit8_slab(s0, minp, maxp, x, c);
-        else limit9_slab(minp, maxp, x, c);
-        ptens = x * dpdissk;
+    double out[2], q0[2] = {0.0, 0.0};
+    if (STAGE == 3) {
+      DvvLane w = d;
+      if (TLDS) wk.get(w);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        pin(y[j]);
+        if constexpr (BIH == 2) q0[j] = (float)div_r(fb[j] * sph_laplacef(ef, df, (float)y[j]), rsph);
+        else if constexpr (BIH == 1) q0[j] = div_r(fb[j] * sph_laplace_tensor(e, w, tv, y[j]), rsph);
+        else q0[j] = div_r(fb[j] * sph_laplace(e, w, y[j]), rsph);
+        pin(q0[j]);
       }
     }
-    if (pt == 0 && son) {
-      if (wmin) ql[0] = minp;
-      if (wmax) ql[QL_MAX] = maxp;
+    fetch(q + 1);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      if (STAGE == 2) qd[j] = y[j];
+      pin(qd[j]);
+      double ptens;
+      if (MIXED) {
+        // flux divergence in FP32 with compensated contractions; the update
+        // qdp - dt*div + qbih stays FP64
+        const double fa = vs0[j] * qd[j], fb2 = vs1[j] * qd[j];
+        const float gv0 = (float)((e.Dinv[0] * fa + e.Dinv[2] * fb2) * e.metdet);
+        const float gv1 = (float)((e.Dinv[1] * fa + e.Dinv[3] * fb2) * e.metdet);
+        const float dv = (row_contractf(df.J, gv0) + col_contractf(df.I, gv1)) * rmd;
+        ptens = (qd[j] + -a.dt * (double)dv + q0[j]);
+      } else {
+        ptens = sph_div_update(e, d, -a.dt, vs0[j], vs1[j], qd[j], q0[j]);
+      }
+      out[j] = ptens;
+      pin(out[j]);
     }
-    if (son) qpo_l[(size_t)q * fs] = (PreT)(e.sph * ptens);
-  };
-  if (GATHER && GD == 2) {
-    PreT gnext[4] = {};
-    if (Q > 1) gq.load(fs, gnext);
-    int q = 0;
-    for (; q + 1 < Q; q += 2) {
-      tracer(q, graw);
-      tracer(q + 1, gnext);
+    if (STAGE == 2) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const double xq = div_r(qd[j], rdp[j]);
+        minp[j] = dmin(minp[j], slab_min(xq));
+        maxp[j] = dmax(maxp[j], slab_max(xq));
+        pin(minp[j]);
+        pin(maxp[j]);
+      }
     }
-    if (q < Q) tracer(q, graw);
-  } else {
-    for (int q = 0; q < Q; ++q) tracer(q, graw);
+    bool moved = false;  // bounds of this lane's levels
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      if (!limit) continue;
+      pin(out[j]);
+      double x = div_r(out[j], rdpd[j]);
+      const double cj = e.sph * rdpd[j].b;
+      const double s0 = slab_sum_serial(x * cj);
+      if (!(s1[j] <= 0)) {
+        if (minp[j] < 0) {
+          minp[j] = 0;
+          moved = true;
+        }
+        if (s0 < minp[j] * s1[j]) {
+          minp[j] = s0 / s1[j];
+          moved = true;
+        }
+        if (s0 > maxp[j] * s1[j]) {
+          maxp[j] = s0 / s1[j];
+          moved = true;
+        }
+        if (a.limiter_option == 8) limit8_slab(s0, minp[j], maxp[j], x, cj);
+        else limit9_slab(minp[j], maxp[j], x, cj);
+        out[j] = x * rdpd[j].b;
+      }
+    }
+    // stage 2 starts from stage 1's bounds; after it they are formed anew
+    if (STAGE == 1 && moved)
+      put_bounds(ql, t, d2_t{minp[0], maxp[0]}, d2_t{minp[1], maxp[1]});
+    typedef typename vec2<PreT>::type V;
+    *(V *)(outE + (size_t)q * fs + oo) = V{(PreT)(e.sph * out[0]), (PreT)(e.sph * out[1])};
   }
 }
 
-// ---------------------------------------------------------------- exchanges
-// The pre-exchange buffers (qdp_pre, qbih_pre, fdss_pre) are stored levels
-// fastest in chunks of 8 levels (lc_index), so a neighbour copy of the 8
-// levels of one GLL point in a chunk is one 64-byte run, half of a line whose
-// other half the same block reads.  An exchange block is one element x one
-// 8-level chunk (XL; 128 lanes, no level padding when the level count is a
-// multiple of 8): lane (pt, kk) gathers point pt at level k0+kk, then the
-// assembled values go through an LDS tile to lanes (kk, pt) and are stored in
-// the slab layout [ie][q][lev][pt].  Blocks walk the elements of one level
-// group in order, so neighbour runs come from L2.
-constexpr int XL = 8;
-constexpr int QB = 8;  // tracers per exchange block
-
-inline int xchg_blocks_x(int nelem, int nlev) {
-  const int nb = nelem * ((nlev + XL - 1) / XL);
-  return (nb + 7) & ~7;
-}
-
-struct XLane {
-  int ie, k0, pt, kk, k;  // gather role: point pt, level k = k0 + kk
-  int wk, wpt;            // store role: level k0 + wk, point wpt
-};
-
-__device__ __forceinline__ bool xchg_lane(int nelem, int nlev, XLane &x) {
-  const int lb = xcd_block(blockIdx.x, gridDim.x);
-  x.ie = lb % nelem;
-  const int g = lb / nelem;
-  x.k0 = g * XL;
-  if (x.k0 >= nlev) return false;  // whole block
-  x.pt = threadIdx.x / XL;
-  x.kk = threadIdx.x % XL;
-  x.k = x.k0 + x.kk;
-  x.wk = threadIdx.x >> 4;
-  x.wpt = threadIdx.x & 15;
-  return true;
-}
-
-
-// DSS of tracers [QB*blockIdx.y, QB*blockIdx.y + QB) and, in the first batch,
-// of the extra field.  avg: stage 3's SSP average (Qdp(n0) + 2 Qdp(np1)) / 3
-// (:379-403) of the assembled tracer value.  F32: the tracer pre-exchange
-// values are FP32 (mixed form), summed in FP64.
-// QMM (stage 2 only): the same block then does euler_qmm_lap_kernel's work on
-// the assembled values in LDS -- the stage-3 bounds (compute_qmin_qmax with
-// rhs_multiplier 2, a.rhs_multiplier set to 2) and the first laplacian of the
-// tracer biharmonic into qbih_pre -- so Qdp(np1) is not read back.
-template <bool F32, bool QMM>
+// The exchange of tracers and extra field, one wave an element's chunk: avg
+// (stage 3) also forms the SSP average (Qdp(n0) + 2 Qdp(np1)) / 3 (:379-403).
+template <bool F32>
 __global__ __launch_bounds__(256) void euler_dss_kernel(EulerArgs a, int avg) {
-  // every assembled field of the block goes into LDS before one barrier
-  __shared__ double tile[QB + 1][XL][17];
-  XLane x;
-  if (!xchg_lane(a.nelem, a.nlev, x)) return;
-  const int L = a.nlev, Q = a.qsize, q0 = blockIdx.y * QB;
-  const int *src = a.src + ((size_t)x.ie * 16 + x.pt) * 3;
-  const int s0 = src[0], s1 = src[1], s2 = src[2];
-  const double r = a.m.rspheremp[(size_t)x.ie * 16 + x.pt];
-  const bool gk = x.k < L, wkv = x.k0 + x.wk < L;
-  const size_t fs = lc_field(L), es = (size_t)Q * fs;
-  const int nq = (Q - q0) < QB ? (Q - q0) : QB;
-  const int kc = gk ? x.k : L - 1;  // gathers of a padding lane stay in bounds
-  // every load of the block's gathers is issued before the first sum
-  double v[QB], fr[4];
+  TLane t;
+  if (!tracer_lane(a.nelem, a.nlev, t)) return;
+  const int L = a.nlev, Q = a.qsize, pt = t.pt;
+  const size_t fs = lc_field(L), es = (size_t)Q * fs, qs = (size_t)L * 16;
+  const double r = a.m.rspheremp[(size_t)t.ie * 16 + pt];
+  const unsigned qo[2] = {(unsigned)(t.lv[0] * 16 + pt), (unsigned)(t.lv[1] * 16 + pt)};
+  if (blockIdx.y == 0) {
+    double x[2];
+    gather_extra(a, a.fdss_pre, t, r, x);
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      if (t.ok[j]) st_stream(&(a.fdss + (size_t)t.ie * qs)[qo[j]], x[j]);
+  }
   using PreT = typename std::conditional<F32, float, double>::type;
-  if (nq > 0) {
+  const double *const avE = avg ? a.qdp_avg_n0 + (size_t)t.ie * Q * qs : nullptr;
+  double *const outE = a.qdp_np1 + (size_t)t.ie * Q * qs;
+  const TGather<PreT> g0((const PreT *)a.qdp_pre, es, t, a.src);
+  // this launch's share of the tracers, QB in flight
+  constexpr int QB = 4;
+  int qa, qb;
+  if (!tracer_share(Q, qa, qb)) return;
+  for (int q = qa; q < qb; q += QB) {
+    TGather<PreT> g[QB] = {g0, g0, g0, g0};
+    double av[QB][2];
 #pragma unroll
-    for (int i = 0; i < QB; ++i)
-      v[i] = gather_lf((const PreT *)a.qdp_pre, es, (size_t)(q0 + (i < nq ? i : 0)) * fs, x.ie, x.pt, kc, s0, s1, s2);
-  }
-  if (q0 == 0) LfGather<double>(a.fdss_pre, fs, x.ie, x.pt, kc, s0, s1, s2).load(0, fr);
-  if (gk) {
+    for (int i = 0; i < QB; ++i) {
+      const size_t qq = q + i < qb ? q + i : qb - 1;
+      g[i].load(qq * fs);
+      if (avg)
 #pragma unroll
-    for (int i = 0; i < QB; ++i)
-      if (i < nq) tile[i][x.kk][x.pt] = v[i] * r;
-    if (q0 == 0) tile[QB][x.kk][x.pt] = gather_sum(fr, s0, s1, s2) * r;
-  }
-  // stage 3: the Qdp(n0) values of the average are loaded before the barrier
-  const size_t o0 = (((size_t)x.ie * Q + q0) * L + x.k0 + x.wk) * 16 + x.wpt, os = (size_t)L * 16;
-  double av[QB];
-  if (avg && wkv && nq > 0) {
+        for (int j = 0; j < 2; ++j) av[i][j] = (avE + qq * qs)[qo[j]];
+    }
 #pragma unroll
-    for (int i = 0; i < QB; ++i) av[i] = a.qdp_avg_n0[o0 + (size_t)(i < nq ? i : 0) * os];
-  }
-  lds_barrier();
-  if (!QMM) {
-    if (wkv) {
+    for (int i = 0; i < QB; ++i) {
+      if (q + i >= qb) break;
 #pragma unroll
-      for (int i = 0; i < QB; ++i) {
-        if (i >= nq) break;
-        double y = tile[i][x.wk][x.wpt];
-        if (avg) y = div_c<3>(av[i] + (3.0 - 1) * y);
-        st_stream(&a.qdp_np1[o0 + (size_t)i * os], y);
+      for (int j = 0; j < 2; ++j) {
+        double y = g[i].sum(j) * r;
+        if (avg) y = div_c<3>(av[i][j] + (3.0 - 1) * y);
+        if (t.ok[j]) st_stream(&(outE + (size_t)(q + i) * qs)[qo[j]], y);
       }
-      if (q0 == 0) st_stream(&a.fdss[((size_t)x.ie * L + x.k0 + x.wk) * 16 + x.wpt], tile[QB][x.wk][x.wpt]);
-    }
-    return;
-  }
-  // stage-3 bounds and first laplacian (euler_qmm_lap_kernel's operations);
-  // every lane of a slab takes part in the cross-lane reductions
-  const int wk = x.k0 + x.wk, wkc = wkv ? wk : L - 1;
-  const size_t sl = ((size_t)x.ie * L + wkc) * 16 + x.wpt;
-  const double rhsmdt = a.rhs_multiplier * a.dt;
-  const double dp = a.derived_dp[sl] - rhsmdt * a.divdp_proj[sl];
-  const double wdp = a.dpdiss_ave[sl];
-  const Recip rdp = recip(dp), rdp0 = recip(a.dp0[wkc]);
-  const bool scale = a.nu_p > 0;
-  ElemLane e;
-  DvvLane d;
-  ElemLaneF ef;
-  DvvLaneF df;
-  if (F32) {
-    load_elemf(a.m, x.ie, x.wpt, ef);
-    load_dvvf(a.m.dvv, x.wpt, df);
-  } else {
-    load_elem_light(a.m, x.ie, x.wpt, e);
-    load_dvv(a.m.dvv, x.wpt, d);
-  }
-  double *ql = a.qlim + ((size_t)x.ie * Q + q0) * ql_row(L) + ql_min(wkc);
-  const size_t ob = ((size_t)x.ie * Q + q0) * fs + lc_index(x.wpt, wkc);
-#pragma unroll
-  for (int i = 0; i < QB; ++i) {
-    if (i >= nq) break;
-    const double y = wkv ? tile[i][x.wk][x.wpt] : 0.0;
-    if (wkv) st_stream(&a.qdp_np1[o0 + (size_t)i * os], y);
-    const double xq = div_r(y, rdp);
-    const double mn = slab_min(xq), mx = slab_max(xq);
-    if (wkv && x.wpt == 0) *(double2 *)(ql + (size_t)i * ql_row(L)) = make_double2(mn, mx);
-    const double yl = scale ? div_r(xq * wdp, rdp0) : xq;
-    if (F32) {
-      const float lap = sph_laplacef(ef, df, (float)yl);
-      if (wkv) ((float *)a.qbih_pre)[ob + (size_t)i * fs] = lap;
-    } else {
-      const double lap = sph_laplace(e, d, yl);
-      if (wkv) a.qbih_pre[ob + (size_t)i * fs] = lap;
     }
   }
-  if (q0 == 0 && wkv) st_stream(&a.fdss[((size_t)x.ie * L + x.k0 + x.wk) * 16 + x.wpt], tile[QB][x.wk][x.wpt]);
 }
 
-// Stage 3 compute_dp + compute_qmin_qmax (rhs_multiplier 2, :406-485) and the
-// first half of the tracer biharmonic (:196-267): laplace(Q * dpdiss_ave / dp0)
-// for every tracer of an (element, level) slab.
-template <bool MIXED>
-__global__ __launch_bounds__(256) void euler_qmm_lap_kernel(EulerArgs a) {
-  size_t slab;
-  int ie, k, pt;
-  if (!slab_ie_k((size_t)a.nelem * a.nlev, a.nlev, slab, ie, k, pt)) return;
-  const int L = a.nlev, Q = a.qsize;
+// The stage-2 exchange with what stage 3 starts from: the assembled Qdp(np1),
+// its bounds (compute_dp + compute_qmin_qmax with rhs_multiplier 2, :406-485)
+// and the first half of the tracer biharmonic, laplace(Q * dpdiss_ave / dp0)
+// (:196-267).  LAP32: FP32 laplacian.
+template <bool PRE32, bool LAP32>
+__global__ __launch_bounds__(256) void euler_dss_lap_kernel(EulerArgs a) {
+  TLane t;
+  if (!tracer_lane(a.nelem, a.nlev, t)) return;
+  const int L = a.nlev, Q = a.qsize, pt = t.pt;
+  const size_t fs = lc_field(L), es = (size_t)Q * fs, qs = (size_t)L * 16;
   ElemLane e;
-  load_elem_light(a.m, ie, pt, e);
+  load_elem_light(a.m, t.ie, pt, e);
   DvvLane d;
-  load_dvv(a.m.dvv, pt, d);
-  const size_t s = slab * 16 + pt;
-  const double rhsmdt = a.rhs_multiplier * a.dt;
-  const double dp = a.derived_dp[s] - rhsmdt * a.divdp_proj[s];
-  const double wdp = a.dpdiss_ave[s];
-  const double dp0 = a.dp0[k];
-  const Recip rdp = recip(dp), rdp0 = recip(dp0);  // shared by the tracers
   ElemLaneF ef;
   DvvLaneF df;
-  if (MIXED) {
-    load_elemf(a.m, ie, pt, ef);
+  if (LAP32) {
+    load_elemf(a.m, t.ie, pt, ef);
     load_dvvf(a.m.dvv, pt, df);
+  } else {
+    load_dvv(a.m.dvv, pt, d);
   }
-  if (Q <= 0) return;
-  // tracer q+1's Qdp is loaded before tracer q's arithmetic
-  const size_t q0i = ((size_t)ie * Q * L + k) * 16 + pt, qs = (size_t)L * 16;
+  const unsigned qo[2] = {(unsigned)(t.lv[0] * 16 + pt), (unsigned)(t.lv[1] * 16 + pt)};
+  double x[2], wdp[2];
+  Recip rdp[2], rdp0[2];
+  gather_extra(a, a.fdss_pre, t, e.rsmp, x);
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const size_t s = (size_t)t.ie * qs + qo[j];
+    if (t.ok[j] && blockIdx.y == 0) st_stream(&a.fdss[s], x[j]);
+    rdp[j] = recip(a.derived_dp[s] - 2.0 * a.dt * a.divdp_proj[s]);
+    rdp0[j] = recip(a.dp0[t.lv[j]]);
+    wdp[j] = a.dpdiss_ave[s];
+  }
+  int qa, qb;
+  if (!tracer_share(Q, qa, qb)) return;
+  using PreT = typename std::conditional<PRE32, float, double>::type;
+  using LapT = typename std::conditional<LAP32, float, double>::type;
   const bool scale = a.nu_p > 0;
-  double nx = a.qdp_n0[q0i];
-  auto tracer = [&](int q) {
-    const double x = div_r(nx, rdp);
-    nx = a.qdp_n0[q0i + (size_t)(q + 1 < Q ? q + 1 : q) * qs];
-    const double mn = slab_min(x), mx = slab_max(x);
-    if (pt == 0) {
-      double *ql = a.qlim + ((size_t)ie * Q + q) * ql_row(L);
-      *(double2 *)(ql + ql_min(k)) = make_double2(mn, mx);
+  double *const outE = a.qdp_np1 + (size_t)t.ie * Q * qs;
+  double *const qlE = a.qlim + (size_t)t.ie * Q * ql_row(L);
+  LapT *const lapE = (LapT *)a.qbih_pre + (size_t)t.ie * es;
+  const unsigned lo = (unsigned)ql_min(t.k0), oo = (unsigned)lc_index(pt, t.k0);
+  TGather<PreT> g((const PreT *)a.qdp_pre, es, t, a.src);
+  g.load((size_t)qa * fs);
+  for (int q = qa; q < qb; ++q) {
+    double y[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) y[j] = g.sum(j) * e.rsmp;
+    g.load((size_t)(q + 1 < qb ? q + 1 : q) * fs);
+    LapT lap[2];
+    d2_t b[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      pin(y[j]);
+      if (t.ok[j]) st_stream(&(outE + (size_t)q * qs)[qo[j]], y[j]);
+      const double xq = div_r(y[j], rdp[j]);
+      b[j] = d2_t{slab_min(xq), slab_max(xq)};
+      const double yl = scale ? div_r(xq * wdp[j], rdp0[j]) : xq;
+      if constexpr (LAP32) lap[j] = sph_laplacef(ef, df, (float)yl);
+      else {
+        lap[j] = sph_laplace(e, d, yl);
+        pin(lap[j]);
+      }
     }
-    const double y = scale ? div_r(x * wdp, rdp0) : x;
-    const size_t o = ((size_t)ie * Q + q) * lc_field(L) + lc_index(pt, k);
-    if (MIXED) ((float *)a.qbih_pre)[o] = sph_laplacef(ef, df, (float)y);
-    else a.qbih_pre[o] = sph_laplace(e, d, y);
-  };
-  // the first tracer is peeled so that on both paths into the loop the same
-  // stores follow the prefetch (the wait then covers the prefetch only)
-  tracer(0);
-  for (int q = 1; q < Q; ++q) tracer(q);
-}
-
-// biharmonic, second half (:216-310): DSS of the first laplacian (with
-// rspheremp), second laplacian, times -rhs_viss*dt*nu_q*dp0/spheremp, for
-// tracers [QB*blockIdx.y, QB*blockIdx.y + QB).  After the LDS transpose the
-// 16-lane groups are slabs (one level, 16 points) for the laplacian.
-template <bool MIXED, bool TENSOR>
-__global__ __launch_bounds__(256) void euler_bih_post_kernel(EulerArgs a) {
-  __shared__ double tile[QB][XL][17];  // every tracer of the block, one barrier
-  XLane x;
-  if (!xchg_lane(a.nelem, a.nlev, x)) return;
-  const int L = a.nlev, Q = a.qsize, q0 = blockIdx.y * QB;
-  const int *src = a.src + ((size_t)x.ie * 16 + x.pt) * 3;
-  const int s0 = src[0], s1 = src[1], s2 = src[2];
-  const bool gk = x.k < L;
-  const int wk = x.k0 + x.wk;
-  const bool wkv = wk < L;
-  const size_t fs = lc_field(L), es = (size_t)Q * fs;
-  const int nq = (Q - q0) < QB ? (Q - q0) : QB;
-  const int kc = gk ? x.k : L - 1;  // gathers of a padding lane stay in bounds
-  // every load of the block's gathers is issued before the first sum
-  double v[QB];
-  {
-    using PreT = typename std::conditional<MIXED, float, double>::type;
-    const LfGather<PreT> g((const PreT *)a.qbih_pre, es, x.ie, x.pt, kc, s0, s1, s2);
-#pragma unroll
-    for (int i = 0; i < QB; ++i) v[i] = g.sum((size_t)(q0 + (i < nq ? i : 0)) * fs, s0, s1, s2);
-  }
-  if (gk) {
-#pragma unroll
-    for (int i = 0; i < QB; ++i)
-      if (i < nq) tile[i][x.kk][x.pt] = v[i];
-  }
-  lds_barrier();
-  // the metric is loaded after the barrier, which the gathers' loads do not
-  // cross: loaded before it, it would be live during them (69 VGPRs instead
-  // of 120 for the FP64 form)
-  ElemLane e;
-  load_elem_light(a.m, x.ie, x.wpt, e);
-  DvvLane d;
-  load_dvv(a.m.dvv, x.wpt, d);
-  ElemLaneF ef;
-  DvvLaneF df;
-  if (MIXED) {
-    load_elemf(a.m, x.ie, x.wpt, ef);
-    load_dvvf(a.m.dvv, x.wpt, df);
-  }
-  double tv[4], vs[6];
-  if (TENSOR) load_tensor(a.m, x.ie, x.wpt, tv, vs);
-  const double f = -a.rhs_viss * a.dt * a.nu_q;
-  const double dp0 = wkv ? a.dp0[wk] : 0.0;
-  const Recip rsph = recip(e.sph);  // shared by the tracers
-#pragma unroll
-  for (int i = 0; i < QB; ++i) {
-    if (i >= nq) break;
-    // every lane of a slab takes part in the laplacian's cross-lane reads
-    const double y = wkv ? tile[i][x.wk][x.wpt] * e.rsmp : 0.0;
-    const size_t o = (((size_t)x.ie * Q + q0 + i) * L + wk) * 16 + x.wpt;
-    if (MIXED) {
-      const double lap = sph_laplacef(ef, df, (float)y);
-      if (wkv) st_stream(&((float *)a.qbih)[o], (float)div_r(f * dp0 * lap, rsph));
-    } else if (TENSOR) {
-      // BIHPostTensorHV (EulerStepFunctorImpl.hpp:281-291)
-      const double lap = sph_laplace_tensor(e, d, tv, y);
-      if (wkv) st_stream(&a.qbih[o], div_r(f * dp0 * lap, rsph));
-    } else {
-      const double lap = sph_laplace(e, d, y);
-      if (wkv) st_stream(&a.qbih[o], div_r(f * dp0 * lap, rsph));
-    }
+    put_bounds(qlE + (size_t)q * ql_row(L) + lo, t, b[0], b[1]);
+    typedef typename vec2<LapT>::type V;
+    *(V *)(lapE + (size_t)q * fs + oo) = V{lap[0], lap[1]};
   }
 }
 
@@ -709,46 +634,26 @@ void launch_euler_nbr_minmax(hipStream_t st, const EulerArgs &a) {
 }
 
 void launch_euler_advect(hipStream_t st, const EulerArgs &a, int stage) {
-  if (a.mixed) hipLaunchKernelGGL((euler_advect_kernel<true, false>), dim3(slab_blocks(a)), dim3(256), 0, st, a, stage);
-  else hipLaunchKernelGGL((euler_advect_kernel<false, false>), dim3(slab_blocks(a)), dim3(256), 0, st, a, stage);
-}
-
-void launch_euler_advect_gather(hipStream_t st, const EulerArgs &a) {
-  const int nb = ((a.nelem * ((a.nlev + AGL - 1) / AGL)) + 7) & ~7;
-  if (a.mixed) hipLaunchKernelGGL((euler_advect_kernel<true, true>), dim3(nb), dim3(16 * AGL), 0, st, a, 2);
-  else hipLaunchKernelGGL((euler_advect_kernel<false, true>), dim3(nb), dim3(16 * AGL), 0, st, a, 2);
+  const dim3 g = tracer_grid(a);
+  auto go = [&](auto *kernel) { hipLaunchKernelGGL(kernel, g, dim3(256), 0, st, a); };
+  if (stage == 1) go(a.mixed ? euler_advect_kernel<true, 1, 0> : euler_advect_kernel<false, 1, 0>);
+  else if (stage == 2) go(a.mixed ? euler_advect_kernel<true, 2, 0> : euler_advect_kernel<false, 2, 0>);
+  else if (a.bih32) go(euler_advect_kernel<true, 3, 2>);
+  else if (a.mixed) go(a.consthv ? euler_advect_kernel<true, 3, 0> : euler_advect_kernel<true, 3, 1>);
+  else go(a.consthv ? euler_advect_kernel<false, 3, 0> : euler_advect_kernel<false, 3, 1>);
 }
 
 void launch_euler_dss(hipStream_t st, const EulerArgs &a, int avg) {
-  const int nq = a.qsize > 0 ? (a.qsize + QB - 1) / QB : 1;
-  const dim3 g(xchg_blocks_x(a.nelem, a.nlev), nq);
-  if (a.mixed) hipLaunchKernelGGL((euler_dss_kernel<true, false>), g, dim3(16 * XL), 0, st, a, avg);
-  else hipLaunchKernelGGL((euler_dss_kernel<false, false>), g, dim3(16 * XL), 0, st, a, avg);
+  const dim3 g(tracer_blocks(a), (a.qsize + 7) / 8 < 1 ? 1 : (a.qsize + 7) / 8);
+  if (a.mixed) hipLaunchKernelGGL(euler_dss_kernel<true>, g, dim3(256), 0, st, a, avg);
+  else hipLaunchKernelGGL(euler_dss_kernel<false>, g, dim3(256), 0, st, a, avg);
 }
 
-bool launch_euler_dss_qmm(hipStream_t st, const EulerArgs &a) {
-  // Used in the mixed form (FP32 pre-exchange values and FP32 biharmonic
-  // buffers), where it measured 1.72 ms against 1.90 for the two launches.
-  // In FP64 the fused kernel (88 VGPRs, 5 waves per SIMD against 7) measured
-  // 2.13 ms against 2.08, so FP64 keeps two launches, as does the mixed form
-  // with tensor hyperviscosity (FP64 biharmonic buffers).
-  if (a.qsize <= 0 || !a.mixed || !a.bih32) return false;
-  const dim3 g(xchg_blocks_x(a.nelem, a.nlev), (a.qsize + QB - 1) / QB);
-  hipLaunchKernelGGL((euler_dss_kernel<true, true>), g, dim3(16 * XL), 0, st, a, 0);
-  return true;
-}
-
-void launch_euler_qmm_lap(hipStream_t st, const EulerArgs &a) {
-  if (a.bih32) hipLaunchKernelGGL(euler_qmm_lap_kernel<true>, dim3(slab_blocks(a)), dim3(256), 0, st, a);
-  else hipLaunchKernelGGL(euler_qmm_lap_kernel<false>, dim3(slab_blocks(a)), dim3(256), 0, st, a);
-}
-
-void launch_euler_bih_post(hipStream_t st, const EulerArgs &a) {
-  if (a.qsize <= 0) return;
-  const dim3 g(xchg_blocks_x(a.nelem, a.nlev), (a.qsize + QB - 1) / QB);
-  if (a.bih32) hipLaunchKernelGGL((euler_bih_post_kernel<true, false>), g, dim3(16 * XL), 0, st, a);
-  else if (a.consthv) hipLaunchKernelGGL((euler_bih_post_kernel<false, false>), g, dim3(16 * XL), 0, st, a);
-  else hipLaunchKernelGGL((euler_bih_post_kernel<false, true>), g, dim3(16 * XL), 0, st, a);
+void launch_euler_dss_lap(hipStream_t st, const EulerArgs &a) {
+  const dim3 g = tracer_grid(a);
+  auto go = [&](auto *kernel) { hipLaunchKernelGGL(kernel, g, dim3(256), 0, st, a); };
+  if (a.bih32) go(euler_dss_lap_kernel<true, true>);
+  else go(a.mixed ? euler_dss_lap_kernel<true, false> : euler_dss_lap_kernel<false, false>);
 }
 
 }  // namespace hx

@@ -101,7 +101,7 @@ struct EulerArgs {
   const double *qdp_n0;       // [ie][q][lev][pt]
   double *qdp_pre;            // pre-DSS output
   double *qdp_np1;            // final output (DSS)
-  double *qbih, *qbih_pre;    // biharmonic buffers
+  double *qbih_pre;           // first laplacian of the biharmonic (FP32 with bih32)
   double *qlim, *qlim_new;    // ql_row / ql_min layout
   const double *derived_dp, *divdp, *divdp_proj, *vn0, *dpdiss_ave, *dpdiss_bih, *dp0;
   double *divdp_w, *divdp_proj_w;
@@ -111,7 +111,7 @@ struct EulerArgs {
   const double *qdp_avg_n0;   // stage 3: Qdp(n0_qdp) for the time average, else nullptr
   const double *qdp_pre_in, *fdss_pre_in;  // stage-1 pre-exchange buffers gathered by the fused stage 2
   int mixed;                  // FP32 flux divergence
-  int bih32;                  // FP32 tracer biharmonic (qbih, qbih_pre hold floats)
+  int bih32;                  // FP32 tracer biharmonic
   int consthv;                // 0: tensor laplacian in the biharmonic's second half
 };
 
@@ -201,13 +201,10 @@ void launch_hv_cycle(hipStream_t st, const HvArgs &a, bool lap1_next);
 void launch_euler_divdp_qmm(hipStream_t st, const EulerArgs &a);
 void launch_euler_nbr_minmax(hipStream_t st, const EulerArgs &a);
 void launch_euler_advect(hipStream_t st, const EulerArgs &a, int stage);
-void launch_euler_advect_gather(hipStream_t st, const EulerArgs &a);
 void launch_euler_dss(hipStream_t st, const EulerArgs &a, int avg);
-// the stage-2 exchange with the stage-3 bounds and first laplacian of the
-// biharmonic (a.rhs_multiplier 2); false: not launched (form not covered)
-bool launch_euler_dss_qmm(hipStream_t st, const EulerArgs &a);
-void launch_euler_qmm_lap(hipStream_t st, const EulerArgs &a);
-void launch_euler_bih_post(hipStream_t st, const EulerArgs &a);
+// the stage-2 exchange with the stage-3 bounds and the first laplacian of the
+// biharmonic
+void launch_euler_dss_lap(hipStream_t st, const EulerArgs &a);
 void launch_state_forcing(hipStream_t st, int nelem, int nlev, double dt, const double *ft, const double *fm,
                           double *t, double *v);
 void launch_tracer_forcing(hipStream_t st, int nelem, int nlev, int qsize, bool moist, double dt, const double *fq,

@@ -87,15 +87,6 @@ __device__ __forceinline__ double slab_sum_serial(double v) {
   return s;
 }
 
-// xor-butterfly within 16 lanes via ds_swizzle (and_mask 0x1F, xor_mask M)
-template <int M>
-__device__ __forceinline__ double xor_get(double x) {
-  constexpr int pattern = 0x1F | (M << 10);
-  const int l = __builtin_amdgcn_ds_swizzle(lo32(x), pattern);
-  const int h = __builtin_amdgcn_ds_swizzle(hi32(x), pattern);
-  return mk64(h, l);
-}
-
 // Division by a divisor shared by many quotients, the same value as a / b
 // (bit for bit, except that a zero quotient may come back as +0): with y = 1/b correctly rounded, q0 = a*y is within one ulp of a/b, the
 // remainder a - q0*b is exact in one FMA, and q0 + rem*y rounded once is the
@@ -136,18 +127,25 @@ __device__ __forceinline__ double vmax64(double a, double b) {
   return r;
 }
 
+// the other lanes' values of a 16-lane reduction whose steps are idempotent:
+// quad_perm [1,0,3,2], [2,3,0,1], then row_half_mirror (the other quad of
+// eight) and row_mirror (the other eight)
+template <int CTRL>
+__device__ __forceinline__ double dpp_get(double x) {
+  return mk64(dpp_mov<CTRL>(hi32(x)), dpp_mov<CTRL>(lo32(x)));
+}
 __device__ __forceinline__ double slab_min(double x) {
-  x = vmin64(x, xor_get<1>(x));
-  x = vmin64(x, xor_get<2>(x));
-  x = vmin64(x, xor_get<4>(x));
-  x = vmin64(x, xor_get<8>(x));
+  x = vmin64(x, dpp_get<0xB1>(x));
+  x = vmin64(x, dpp_get<0x4E>(x));
+  x = vmin64(x, dpp_get<0x141>(x));
+  x = vmin64(x, dpp_get<0x140>(x));
   return x;
 }
 __device__ __forceinline__ double slab_max(double x) {
-  x = vmax64(x, xor_get<1>(x));
-  x = vmax64(x, xor_get<2>(x));
-  x = vmax64(x, xor_get<4>(x));
-  x = vmax64(x, xor_get<8>(x));
+  x = vmax64(x, dpp_get<0xB1>(x));
+  x = vmax64(x, dpp_get<0x4E>(x));
+  x = vmax64(x, dpp_get<0x141>(x));
+  x = vmax64(x, dpp_get<0x140>(x));
   return x;
 }
 
