@@ -380,12 +380,16 @@ static void launch_caar_as(hipStream_t st, const CaarArgs &a) {
   const dim3 threads((nch * 16 + 63) & ~63);  // at most 1024 (REMAP_MAX_NLEV levels)
   const size_t lds = ((size_t)3 * caar_rows<CL>(a.nlev) + (RS0 ? 1 : 0)) * 16 * sizeof(double);
   auto go = [&](auto *kernel) { hipLaunchKernelGGL(kernel, dim3(a.nelem), threads, lds, st, a); };
-  // six levels per lane and rsplit == 0 hold more (168 VGPRs), which blocks of
-  // up to 512 lanes may
+  // six levels per lane (up to 96 levels: 256 lanes) and rsplit == 0 hold more
+  // (168 VGPRs), which blocks of up to 512 lanes may
   constexpr int T = RS0 || CL > 4 ? 512 : 1024;
-  if (threads.x > T)
-    go(a.qdp_n0 ? caar_kernel<CL, RS0, GATHER, BASE, true, 1024> : caar_kernel<CL, RS0, GATHER, BASE, false, 1024>);
-  else go(a.qdp_n0 ? caar_kernel<CL, RS0, GATHER, BASE, true, T> : caar_kernel<CL, RS0, GATHER, BASE, false, T>);
+  if constexpr (RS0) {
+    if (threads.x > T) {
+      go(a.qdp_n0 ? caar_kernel<CL, RS0, GATHER, BASE, true, 1024> : caar_kernel<CL, RS0, GATHER, BASE, false, 1024>);
+      return;
+    }
+  }
+  go(a.qdp_n0 ? caar_kernel<CL, RS0, GATHER, BASE, true, T> : caar_kernel<CL, RS0, GATHER, BASE, false, T>);
 }
 
 template <int CL>
