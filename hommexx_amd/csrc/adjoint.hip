@@ -588,14 +588,22 @@ __global__ __launch_bounds__(64) void adj_remap_grid_kernel(AdjRemapArgs a) {
   for (int k = 0; k < L; ++k) ps += src(k);
   ps += a.hyai[0] * a.ps0;
   double acc = 0.0, accn = 0.0;
-  for (int k = 0; k < L; ++k) {
-    const double tg = (a.hyai[k + 1] - a.hyai[k]) * a.ps0 + (a.hybi[k + 1] - a.hybi[k]) * ps;
-    c.g(RG_TG, k) = tg;
-    c.g(RG_PIO, k) = acc;
-    pio_s[k * bs + tid] = acc;
-    c.g(RG_PIN, k) = accn;
-    acc += src(k);
-    accn += tg;
+  for (int b = 0; b < L; b += 8) {  // (loads ahead of the stores, which may alias them)
+    double x[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = src(b + i < L ? b + i : L - 1);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int k = b + i;
+      if (k >= L) break;
+      const double tg = (a.hyai[k + 1] - a.hyai[k]) * a.ps0 + (a.hybi[k + 1] - a.hybi[k]) * ps;
+      c.g(RG_TG, k) = tg;
+      c.g(RG_PIO, k) = acc;
+      pio_s[k * bs + tid] = acc;
+      c.g(RG_PIN, k) = accn;
+      acc += x[i];
+      accn += tg;
+    }
   }
   const double pioL = acc;  // pio(L-1) + dx(L-1)
   c.g(RG_PIO, L) = pioL;
@@ -619,117 +627,208 @@ __global__ __launch_bounds__(64) void adj_remap_grid_kernel(AdjRemapArgs a) {
   }
 }
 
-// one lane = (column, field): forward recompute of the field's PPM
-// reconstruction, then the reverse sweep; per-field grid adjoints go to
-// scratch for adj_remap_finish_kernel
-__global__ __launch_bounds__(256) void adj_remap_field_kernel(AdjRemapArgs a) {
+// The fields' part: forward recompute of the PPM reconstruction, then the reverse
+// sweep; per-field grid adjoints go to scratch for adj_remap_finish_kernel.
+//
+// Bound: latency of a column's serial passes.  One lane per (column, field) ran
+// them all in one kernel (73728 lanes at 1536 elements: a wave per SIMD, every
+// load exposed): 1141 us there at L72, 679 at 384 elements.  Only three of
+// the sums along a column are chains (the mass prefix, its reverse, and the
+// totals of a source cell); the others reach at most three levels.  So a
+// lane is (ADJ_CH scratch entries, column, field) and owns the entries [i0, i1)
+// of every array; each pass starts as many levels earlier as its window
+// reaches, in the same order, and stores only its own entries: the same
+// values bit for bit, with a launch per dependence between chunks.  The two mass
+// scans are an extra chunk of the passes beside them.
+// Now, us at 1536 and 384 elements L72: forward 156, 44; targets 209, 57; cells 88,
+// 18; interfaces 100, 25; slopes 73, 26; values 48, 14: 674 and 184 in all.  Chunks
+// of 4, 16 and 24 entries: 725, 666, 659 and 197, 237, 284 (before the scans'
+// loads were batched).
+constexpr int ADJ_CH = 8;
+static int adj_chunks(int nlev) { return (nlev + 4 + ADJ_CH - 1) / ADJ_CH; }
+
+struct RField {
+  const AdjRemapArgs *a;
+  RCol c;
+  int L, fld, ie, pt, chunk, i0, i1;
+  const double *fin;
+  double *lam;
+  __device__ __forceinline__ double src(int k) const { return a->dp[((size_t)ie * L + k) * 16 + pt]; }
+  __device__ __forceinline__ double DX(int i) const { return src(ghost_src(i, L)); }
+  __device__ __forceinline__ size_t fidx(int k) const {
+    return fld < 2 ? (((size_t)ie * L + k) * 2 + fld) * 16 + pt : ((size_t)ie * L + k) * 16 + pt;
+  }
+  __device__ __forceinline__ double &F(int arr, int i) const { return c.f(fld, arr, i); }
+  __device__ __forceinline__ double &A(int j) const { return F(RF_AA, j + 1); }  // a(j), j = -1..L+2
+  __device__ __forceinline__ double &LA(int j) const { return F(RF_LA, j + 1); }
+  __device__ __forceinline__ bool own(int i) const { return i >= i0 && i < i1; }
+};
+
+__device__ __forceinline__ bool remap_lane(const AdjRemapArgs &a, RField &f) {
   const size_t ncol = (size_t)a.nelem * 16;
   const size_t lane = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (lane >= 3 * ncol) return;
-  const int fld = (int)(lane / ncol);
+  if (lane >= 3 * ncol) return false;
   const size_t col = lane % ncol;
-  const int L = a.nlev, ie = (int)(col >> 4), pt = (int)(col & 15);
-  const RCol c{&a, col, ncol, (size_t)L + 4};
-  auto src = [&](int k) { return a.dp[((size_t)ie * L + k) * 16 + pt]; };
-  auto DX = [&](int i) { return src(ghost_src(i, L)); };
-  auto fidx = [&](int k) {
-    return fld < 2 ? (((size_t)ie * L + k) * 2 + fld) * 16 + pt : ((size_t)ie * L + k) * 16 + pt;
-  };
-  const double *fin = fld < 2 ? a.v : a.t;
-  double *lam = fld < 2 ? a.l_v : a.l_t;
-  auto F = [&](int arr, int i) -> double & { return c.f(fld, arr, i); };
-  auto A = [&](int j) -> double & { return F(RF_AA, j + 1); };   // a(j), j = -1..L+2
-  auto LA = [&](int j) -> double & { return F(RF_LA, j + 1); };
-  const int W = L + 4;
+  f.a = &a;
+  f.L = a.nlev;
+  f.c = RCol{&a, col, ncol, (size_t)a.nlev + 4};
+  f.fld = (int)(lane / ncol);
+  f.ie = (int)(col >> 4);
+  f.pt = (int)(col & 15);
+  f.chunk = blockIdx.y;
+  f.i0 = f.chunk * ADJ_CH;
+  f.i1 = f.i0 + ADJ_CH < f.L + 4 ? f.i0 + ADJ_CH : f.L + 4;
+  f.fin = f.fld < 2 ? a.v : a.t;
+  f.lam = f.fld < 2 ? a.l_v : a.l_t;
+  return true;
+}
+
+// parabola of cell j (1..L): flags and coefficients
+struct Parabola {
+  double c0, c1, c2;
+  bool flat, f2, f3, bnd;
+};
+__device__ __forceinline__ Parabola parabola(const RField &f, int j) {
+  Parabola p;
+  const double al0 = f.F(RF_AI, j - 1), ar0 = f.F(RF_AI, j), aa = f.A(j);
+  p.flat = (ar0 - aa) * (aa - al0) <= 0.0;
+  double al = p.flat ? aa : al0, ar = p.flat ? aa : ar0;
+  p.f2 = (ar - al) * (aa - (al + ar) / 2.0) > (ar - al) * (ar - al) / 6.0;
+  if (p.f2) al = 3.0 * aa - 2.0 * ar;
+  p.f3 = (ar - al) * (aa - (al + ar) / 2.0) < -(ar - al) * (ar - al) / 6.0;
+  if (p.f3) ar = 3.0 * aa - 2.0 * al;
+  p.c0 = 1.5 * aa - (al + ar) / 4.0;
+  p.c1 = ar - al;
+  p.c2 = 3.0 * (-2.0 * aa + (al + ar));
+  p.bnd = f.a->alg == 2 && (j <= 2 || j >= f.L - 1);
+  if (p.bnd) { p.c0 = aa; p.c1 = 0.0; p.c2 = 0.0; }
+  return p;
+}
+
+// a, dma, ai; the extra chunk: the mass above each cell (RF_LD, which the reverse
+// passes write only after its last use)
+__global__ __launch_bounds__(256) void adj_remap_forward_kernel(AdjRemapArgs a) {
+  RField f;
+  if (!remap_lane(a, f)) return;
+  const int L = f.L;
+  if (f.i0 >= L + 4) {
+    double prefix = 0.0;
+    for (int b = 0; b < L; b += 8) {  // (loads ahead of the stores, which may alias them)
+      double x[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int j = b + i < L ? b + i : L - 1;
+        x[i] = f.fin[f.fidx(j)] * f.src(j);
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if (b + i >= L) break;
+        f.F(RF_LD, b + i) = prefix;
+        prefix += x[i];
+      }
+    }
+    return;
+  }
   // sums over the targets of a source cell: cells without targets stay zero
-  for (int i = 0; i < W; ++i) {
-    F(RF_LC0, i) = 0.0; F(RF_LC1, i) = 0.0; F(RF_LC2, i) = 0.0; F(RF_LMASS, i) = 0.0; F(RF_LDX, i) = 0.0;
-    F(RF_LPIO, i) = 0.0; F(RF_LPIN, i) = 0.0;
+  for (int i = f.i0; i < f.i1; ++i) {
+    f.F(RF_LC0, i) = 0.0; f.F(RF_LC1, i) = 0.0; f.F(RF_LC2, i) = 0.0; f.F(RF_LMASS, i) = 0.0; f.F(RF_LDX, i) = 0.0;
+    f.F(RF_LPIO, i) = 0.0; f.F(RF_LPIN, i) = 0.0;
   }
-  // ---------------------------------------------------------- forward
-  for (int k = 0; k < L; ++k) {
-    const double x = src(k);
-    A(k + 1) = (fin[fidx(k)] * x) / x;
-  }
-  A(0) = A(1); A(-1) = A(2); A(L + 1) = A(L); A(L + 2) = A(L - 1);
-  double X[4], dG[4];
-  for (int j = 0; j < L + 2; ++j) {
-    for (int m = 0; m < 4; ++m) X[m] = DX(j + m < L + 3 ? j + m : L + 3);
+  auto a_of = [&](int j) {  // j = -1..L+2, mirrored ghosts
+    const int k = j < 1 ? -j : j > L ? 2 * L - j : j - 1;
+    const double x = f.src(k);
+    return (f.fin[f.fidx(k)] * x) / x;
+  };
+  auto dma_of = [&](int j, double am, double a0, double ap) {
+    double X[4], dG[4];
+    for (int m = 0; m < 4; ++m) X[m] = f.DX(j + m < L + 3 ? j + m : L + 3);
     const double g0 = ppm_g(0, X, dG), g1 = ppm_g(1, X, dG), g2 = ppm_g(2, X, dG);
-    const double dp_ = A(j + 1) - A(j), dm_ = A(j) - A(j - 1);
+    const double dp_ = ap - a0, dm_ = a0 - am;
     double dma = 0.0;
     if (dp_ * dm_ > 0.0) {
       const double da = g0 * (g1 * dp_ + g2 * dm_);
       const double bc = 2.0 * fabs(dm_) < 2.0 * fabs(dp_) ? 2.0 * fabs(dm_) : 2.0 * fabs(dp_);
       dma = (fabs(da) < bc ? fabs(da) : bc) * copysign(1.0, da);
     }
-    F(RF_DMA, j) = dma;
-  }
-  for (int j = 0; j < L + 1; ++j) {
-    for (int m = 0; m < 4; ++m) X[m] = DX(j + m);
-    double gg[10];
-    for (int i = 3; i < 10; ++i) gg[i] = ppm_g(i, X, dG);
-    const double d1 = A(j + 1) - A(j);
-    F(RF_AI, j) = A(j) + gg[3] * d1 +
-                  gg[4] * (gg[5] * (gg[6] - gg[7]) * d1 - gg[8] * F(RF_DMA, j + 1) + gg[9] * F(RF_DMA, j));
-  }
-  // parabola of cell j (1..L): flags and coefficients
-  auto parabola = [&](int j, double &c0, double &c1, double &c2, bool &flat, bool &f2, bool &f3, bool &bnd) {
-    const double al0 = F(RF_AI, j - 1), ar0 = F(RF_AI, j), aa = A(j);
-    flat = (ar0 - aa) * (aa - al0) <= 0.0;
-    double al = flat ? aa : al0, ar = flat ? aa : ar0;
-    f2 = (ar - al) * (aa - (al + ar) / 2.0) > (ar - al) * (ar - al) / 6.0;
-    if (f2) al = 3.0 * aa - 2.0 * ar;
-    f3 = (ar - al) * (aa - (al + ar) / 2.0) < -(ar - al) * (ar - al) / 6.0;
-    if (f3) ar = 3.0 * aa - 2.0 * al;
-    c0 = 1.5 * aa - (al + ar) / 4.0;
-    c1 = ar - al;
-    c2 = 3.0 * (-2.0 * aa + (al + ar));
-    bnd = a.alg == 2 && (j <= 2 || j >= L - 1);
-    if (bnd) { c0 = aa; c1 = 0.0; c2 = 0.0; }
+    return dma;
   };
-  // The reverse passes accumulate in registers over a sliding window of
-  // levels and write each scratch entry once (or add to it once), so no
-  // entry is read back while its own update is still in flight.
-  // ------------------------------------------ reverse: targets (ascending)
-  // kid is non-decreasing in k: the targets of one source cell are
-  // consecutive, and the cell's sums are written when the cell changes
-  double prefix = 0.0, mprev = 0.0;
-  int jj = 0, cur = -1;
+  // entry i of RF_AA is a(i - 1); dma(j) and ai(j) are entries j
+  double am = a_of(f.i0 - 1), a0 = f.i0 <= L + 2 ? a_of(f.i0) : 0.0, dcur = 0.0;
+  if (f.i0 <= L + 1) dcur = dma_of(f.i0, am, a0, a_of(f.i0 + 1));
+  for (int j = f.i0; j < f.i1; ++j) {
+    f.A(j - 1) = am;
+    if (j > L + 1) {
+      am = a0;
+      a0 = j + 1 <= L + 2 ? a_of(j + 1) : 0.0;
+      continue;
+    }
+    f.F(RF_DMA, j) = dcur;
+    const double ap = a_of(j + 1);
+    if (j <= L) {
+      const double dnext = dma_of(j + 1, a0, ap, a_of(j + 2));
+      double X[4], dG[4], gg[10];
+      for (int m = 0; m < 4; ++m) X[m] = f.DX(j + m);
+      for (int i = 3; i < 10; ++i) gg[i] = ppm_g(i, X, dG);
+      const double d1 = ap - a0;
+      f.F(RF_AI, j) = a0 + gg[3] * d1 + gg[4] * (gg[5] * (gg[6] - gg[7]) * d1 - gg[8] * dnext + gg[9] * dcur);
+      dcur = dnext;
+    }
+    am = a0;
+    a0 = ap;
+  }
+}
+
+// reverse, targets (ascending): kid is non-decreasing in k, so the targets of one
+// source cell are consecutive; a lane takes the targets of its own cells, and of
+// the cell above them, whose last sum reaches into its first entry
+__global__ __launch_bounds__(256) void adj_remap_target_kernel(AdjRemapArgs a) {
+  RField f;
+  if (!remap_lane(a, f)) return;
+  const int L = f.L;
+  int lo = 0, hi = L;  // the first target of cell i0 - 1 or a later one
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if ((int)f.c.g(RG_KID, mid) < f.i0 - 1) lo = mid + 1;
+    else hi = mid;
+  }
+  if (lo >= L) return;
+  const int ks = lo > 0 ? lo - 1 : 0;  // (the one before: its mass)
+  double mprev = 0.0;
+  int cur = -1;
   double s_lc0 = 0.0, s_lc1 = 0.0, s_lc2 = 0.0, s_lm = 0.0, s_ldx = 0.0, s_plo = 0.0, s_phi = 0.0;
   auto flush_cell = [&]() {
     if (cur < 0) return;
-    F(RF_LC0, cur) = s_lc0;
-    F(RF_LC1, cur) = s_lc1;
-    F(RF_LC2, cur) = s_lc2;
-    F(RF_LMASS, cur) = s_lm;
-    F(RF_LDX, cur) = s_ldx;
-    F(RF_LPIO, cur) += s_plo;
-    F(RF_LPIO, cur + 1) += s_phi;
+    if (f.own(cur)) {
+      f.F(RF_LC0, cur) = s_lc0;
+      f.F(RF_LC1, cur) = s_lc1;
+      f.F(RF_LC2, cur) = s_lc2;
+      f.F(RF_LMASS, cur) = s_lm;
+      f.F(RF_LDX, cur) = s_ldx;
+      f.F(RF_LPIO, cur) += s_plo;
+    }
+    if (f.own(cur + 1)) f.F(RF_LPIO, cur + 1) += s_phi;
   };
-  double lcur = lam[fidx(0)] / c.g(RG_TG, 0);
-  for (int k = 0; k < L; ++k) {
-    const int kk = (int)c.g(RG_KID, k);
+  double lcur = f.lam[f.fidx(ks)] / f.c.g(RG_TG, ks);
+  for (int k = ks; k < L; ++k) {
+    const int kk = (int)f.c.g(RG_KID, k);
+    if (kk >= f.i1) break;
     if (kk != cur) {
       flush_cell();
       cur = kk;
       s_lc0 = s_lc1 = s_lc2 = s_lm = s_ldx = s_plo = s_phi = 0.0;
     }
-    while (jj < kk) { prefix += fin[fidx(jj)] * src(jj); ++jj; }
-    const double z2 = c.g(RG_Z2, k), dxk = src(kk), tg = c.g(RG_TG, k);
-    double c0, c1, c2; bool fl, f2, f3, bd;
-    parabola(kk + 1, c0, c1, c2, fl, f2, f3, bd);
-    const double integ = (c0 * (z2 + 0.5) + c1 * (z2 * z2 - 0.25) / 2.0) + c2 * (z2 * z2 * z2 + 0.125) / 3.0;
-    const double m = prefix + integ * dxk;
+    const double z2 = f.c.g(RG_Z2, k), dxk = f.src(kk), tg = f.c.g(RG_TG, k);
+    const Parabola p = parabola(f, kk + 1);
+    const double integ = (p.c0 * (z2 + 0.5) + p.c1 * (z2 * z2 - 0.25) / 2.0) + p.c2 * (z2 * z2 * z2 + 0.125) / 3.0;
+    const double m = f.F(RF_LD, kk) + integ * dxk;
     const double out = k > 0 ? m - mprev : m;
     mprev = m;
-    const double lf = lam[fidx(k)];
-    F(RF_LTG, k) = -lf * (out / tg) / tg;
-    const double lnext = k + 1 < L ? lam[fidx(k + 1)] / c.g(RG_TG, k + 1) : 0.0;
+    const double lf = f.lam[f.fidx(k)];
+    const double lnext = k + 1 < L ? f.lam[f.fidx(k + 1)] / f.c.g(RG_TG, k + 1) : 0.0;
     const double lm = lcur - lnext;
     lcur = lnext;
     const double li = lm * dxk;
-    const double lz2 = li * (c0 + c1 * z2 + c2 * z2 * z2);
+    const double lz2 = li * (p.c0 + p.c1 * z2 + p.c2 * z2 * z2);
     s_lm += lm;
     s_ldx += lm * integ - lz2 * z2 / dxk;
     s_lc0 += li * (z2 + 0.5);
@@ -737,127 +836,175 @@ __global__ __launch_bounds__(256) void adj_remap_field_kernel(AdjRemapArgs a) {
     s_lc2 += li * (z2 * z2 * z2 + 0.125) / 3.0;
     s_plo -= 0.5 * lz2 / dxk;
     s_phi -= 0.5 * lz2 / dxk;
-    F(RF_LPIN, k + 1) = lz2 / dxk;
-  }
-  flush_cell();
-  // mass prefix -> lambda of var: LMASS(j) becomes sum_{i > j} LMASS(i)
-  {
-    double s = F(RF_LMASS, L);
-    for (int j = L - 1; j >= 0; --j) {
-      const double o = F(RF_LMASS, j);
-      F(RF_LMASS, j) = s;
-      s += o;
+    if (f.own(kk)) {
+      f.F(RF_LTG, k) = -lf * (out / tg) / tg;
+      f.F(RF_LPIN, k + 1) = lz2 / dxk;
     }
   }
-  // cells (descending): coefficients -> a(j), ai(j-1), ai(j); first writer of
-  // LAI (all) and LA(1..L)
-  LA(-1) = 0.0; LA(0) = 0.0; LA(L + 1) = 0.0; LA(L + 2) = 0.0;
+  flush_cell();
+}
+
+// reverse, cells (descending): coefficients -> a(j), ai(j-1), ai(j); first writer
+// of LAI (all) and LA.  The extra chunk: mass prefix -> lambda of var, LMASS(j)
+// becomes sum_{i > j} LMASS(i)
+__global__ __launch_bounds__(256) void adj_remap_cell_kernel(AdjRemapArgs a) {
+  RField f;
+  if (!remap_lane(a, f)) return;
+  const int L = f.L;
+  if (f.i0 >= L + 4) {
+    double s = f.F(RF_LMASS, L);
+    for (int b = L - 1; b >= 0; b -= 8) {
+      double x[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = f.F(RF_LMASS, b - i > 0 ? b - i : 0);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if (b < i) break;
+        f.F(RF_LMASS, b - i) = s;
+        s += x[i];
+      }
+    }
+    return;
+  }
+  if (f.chunk == 0) f.LA(-1) = 0.0, f.LA(0) = 0.0, f.LA(L + 1) = 0.0, f.LA(L + 2) = 0.0;
   double lai_carry = 0.0;  // ai(j) as the left edge of cell j+1
-  for (int j = L; j >= 1; --j) {
+  for (int j = f.i1 < L ? f.i1 : L; j >= 1 && j >= f.i0; --j) {
     const int cidx = j - 1;
-    double c0, c1, c2; bool flat, f2, f3, bnd;
-    parabola(j, c0, c1, c2, flat, f2, f3, bnd);
-    const double l0 = F(RF_LC0, cidx), l1 = F(RF_LC1, cidx), l2 = F(RF_LC2, cidx);
+    const Parabola p = parabola(f, j);
+    const double l0 = f.F(RF_LC0, cidx), l1 = f.F(RF_LC1, cidx), l2 = f.F(RF_LC2, cidx);
     double laa, lal, lar;
-    if (bnd) {
+    if (p.bnd) {
       laa = l0; lal = 0.0; lar = 0.0;
     } else {
       laa = 1.5 * l0 - 6.0 * l2;
       lal = -l0 / 4.0 - l1 + 3.0 * l2;
       lar = -l0 / 4.0 + l1 + 3.0 * l2;
-      if (f3) { laa += 3.0 * lar; lal += -2.0 * lar; lar = 0.0; }
-      if (f2) { laa += 3.0 * lal; lar += -2.0 * lal; lal = 0.0; }
-      if (flat) { laa += lal + lar; lal = 0.0; lar = 0.0; }
+      if (p.f3) { laa += 3.0 * lar; lal += -2.0 * lar; lar = 0.0; }
+      if (p.f2) { laa += 3.0 * lal; lar += -2.0 * lal; lal = 0.0; }
+      if (p.flat) { laa += lal + lar; lal = 0.0; lar = 0.0; }
     }
-    F(RF_LAI, j) = lai_carry + lar;
+    if (f.own(j)) {
+      f.F(RF_LAI, j) = lai_carry + lar;
+      f.LA(j) = laa;
+    }
     lai_carry = lal;
-    LA(j) = laa;
   }
-  F(RF_LAI, 0) = lai_carry;
-  // interfaces ai(j), j = L..0; first writer of LDMA and LD
-  {
-    double la_carry = 0.0, ldma_carry = 0.0, w[4] = {0.0, 0.0, 0.0, 0.0};  // w[m]: LD(j+m)
-    for (int j = L; j >= 0; --j) {
-      if (j + 4 <= L + 3) F(RF_LD, j + 4) = w[3];
-      w[3] = w[2]; w[2] = w[1]; w[1] = w[0]; w[0] = 0.0;
-      for (int m = 0; m < 4; ++m) X[m] = DX(j + m);
-      double gg[10], dd[10][4];
-      for (int i = 3; i < 10; ++i) gg[i] = ppm_g(i, X, dd[i]);
-      const double li = F(RF_LAI, j);
-      const double d1 = A(j + 1) - A(j);
-      const double g56 = gg[5] * (gg[6] - gg[7]);
-      const double dmaj = F(RF_DMA, j), dmaj1 = F(RF_DMA, j + 1);
-      const double ld1 = li * (gg[3] + gg[4] * g56);
-      LA(j + 1) += la_carry + ld1;
-      la_carry = li - ld1;
-      F(RF_LDMA, j + 1) = ldma_carry - li * gg[4] * gg[8];
-      ldma_carry = li * gg[4] * gg[9];
-      double lg[10] = {0};
-      lg[3] = li * d1;
-      lg[4] = li * (g56 * d1 - gg[8] * dmaj1 + gg[9] * dmaj);
-      const double lg56 = li * gg[4] * d1;
-      lg[5] = lg56 * (gg[6] - gg[7]);
-      lg[6] = lg56 * gg[5];
-      lg[7] = -lg56 * gg[5];
-      lg[8] = -li * gg[4] * dmaj1;
-      lg[9] = li * gg[4] * dmaj;
-      for (int i = 3; i < 10; ++i)
-        for (int m = 0; m < 4; ++m) w[m] += lg[i] * dd[i][m];
+  if (f.chunk == 0) f.F(RF_LAI, 0) = lai_carry;
+}
+
+// reverse, interfaces ai(j), j = L..0; first writer of LDMA and LD
+__global__ __launch_bounds__(256) void adj_remap_interface_kernel(AdjRemapArgs a) {
+  RField f;
+  if (!remap_lane(a, f)) return;
+  const int L = f.L;
+  double X[4];
+  double la_carry = 0.0, ldma_carry = 0.0, w[4] = {0.0, 0.0, 0.0, 0.0};  // w[m]: LD(j+m)
+  const int first = f.i1 - 1 < L ? f.i1 - 1 : L, last = f.i0 > 3 ? f.i0 - 3 : 0;
+  for (int j = first; j >= last; --j) {
+    if (f.own(j + 4)) f.F(RF_LD, j + 4) = w[3];
+    w[3] = w[2]; w[2] = w[1]; w[1] = w[0]; w[0] = 0.0;
+    for (int m = 0; m < 4; ++m) X[m] = f.DX(j + m);
+    double gg[10], dd[10][4];
+#pragma unroll
+    for (int i = 3; i < 10; ++i) gg[i] = ppm_g(i, X, dd[i]);
+    const double li = f.F(RF_LAI, j);
+    const double d1 = f.A(j + 1) - f.A(j);
+    const double g56 = gg[5] * (gg[6] - gg[7]);
+    const double dmaj = f.F(RF_DMA, j), dmaj1 = f.F(RF_DMA, j + 1);
+    const double ld1 = li * (gg[3] + gg[4] * g56);
+    if (f.own(j + 1)) {
+      f.LA(j + 1) += la_carry + ld1;
+      f.F(RF_LDMA, j + 1) = ldma_carry - li * gg[4] * gg[8];
     }
-    LA(0) += la_carry;
-    F(RF_LDMA, 0) = ldma_carry;
-    for (int m = 0; m < 4; ++m) F(RF_LD, m) = w[m];
+    la_carry = li - ld1;
+    ldma_carry = li * gg[4] * gg[9];
+    double lg[10] = {0};
+    lg[3] = li * d1;
+    lg[4] = li * (g56 * d1 - gg[8] * dmaj1 + gg[9] * dmaj);
+    const double lg56 = li * gg[4] * d1;
+    lg[5] = lg56 * (gg[6] - gg[7]);
+    lg[6] = lg56 * gg[5];
+    lg[7] = -lg56 * gg[5];
+    lg[8] = -li * gg[4] * dmaj1;
+    lg[9] = li * gg[4] * dmaj;
+#pragma unroll
+    for (int i = 3; i < 10; ++i)
+#pragma unroll
+      for (int m = 0; m < 4; ++m) w[m] += lg[i] * dd[i][m];
   }
-  // dma(j), j = L+1..0
-  {
-    double c1 = 0.0, c2 = 0.0, w[3] = {0.0, 0.0, 0.0};  // c1: LA(j+1) pending, c2: LA(j); w[m]: LD(j+m)
-    for (int j = L + 1; j >= 0; --j) {
-      if (j + 3 <= L + 3) F(RF_LD, j + 3) += w[2];
-      w[2] = w[1]; w[1] = w[0]; w[0] = 0.0;
-      double ldp = 0.0, ldm = 0.0;
-      const double dp_ = A(j + 1) - A(j), dm_ = A(j) - A(j - 1);
-      if (dp_ * dm_ > 0.0) {
-        for (int m = 0; m < 4; ++m) X[m] = DX(j + m < L + 3 ? j + m : L + 3);
-        double d0[4], d1[4], d2[4];
-        const double g0 = ppm_g(0, X, d0), g1 = ppm_g(1, X, d1), g2 = ppm_g(2, X, d2);
-        const double da = g0 * (g1 * dp_ + g2 * dm_);
-        const bool bsel = 2.0 * fabs(dm_) < 2.0 * fabs(dp_);
-        const double bc = bsel ? 2.0 * fabs(dm_) : 2.0 * fabs(dp_);
-        const bool asel = fabs(da) < bc;
-        const double sda = da > 0.0 ? 1.0 : da < 0.0 ? -1.0 : 0.0;
-        const double lm3 = F(RF_LDMA, j) * sda;
-        double lda = 0.0;
-        if (asel) {
-          lda = lm3 * sda;
-        } else if (bsel) {
-          ldm = 2.0 * (dm_ > 0.0 ? 1.0 : dm_ < 0.0 ? -1.0 : 0.0) * lm3;
-        } else {
-          ldp = 2.0 * (dp_ > 0.0 ? 1.0 : dp_ < 0.0 ? -1.0 : 0.0) * lm3;
-        }
-        const double lg0 = lda * (g1 * dp_ + g2 * dm_), lg1 = lda * g0 * dp_, lg2 = lda * g0 * dm_;
-        ldp += lda * g0 * g1;
-        ldm += lda * g0 * g2;
-        for (int m = 0; m < 3; ++m) w[m] += lg0 * d0[m] + lg1 * d1[m] + lg2 * d2[m];
+  if (f.chunk == 0) {
+    f.LA(0) += la_carry;
+    f.F(RF_LDMA, 0) = ldma_carry;
+  }
+#pragma unroll
+  for (int m = 0; m < 4; ++m)
+    if (f.own(last + m)) f.F(RF_LD, last + m) = w[m];
+}
+
+// reverse, dma(j), j = L+1..0
+__global__ __launch_bounds__(256) void adj_remap_slope_kernel(AdjRemapArgs a) {
+  RField f;
+  if (!remap_lane(a, f)) return;
+  const int L = f.L;
+  double X[4];
+  double c1 = 0.0, c2 = 0.0, w[3] = {0.0, 0.0, 0.0};  // c1: LA(j+1) pending, c2: LA(j); w[m]: LD(j+m)
+  const int first = f.i1 < L + 1 ? f.i1 : L + 1, last = f.i0 > 2 ? f.i0 - 2 : 0;
+  for (int j = first; j >= last; --j) {
+    if (f.own(j + 3)) f.F(RF_LD, j + 3) += w[2];
+    w[2] = w[1]; w[1] = w[0]; w[0] = 0.0;
+    double ldp = 0.0, ldm = 0.0;
+    const double dp_ = f.A(j + 1) - f.A(j), dm_ = f.A(j) - f.A(j - 1);
+    if (dp_ * dm_ > 0.0) {
+      for (int m = 0; m < 4; ++m) X[m] = f.DX(j + m < L + 3 ? j + m : L + 3);
+      double d0[4], d1[4], d2[4];
+      const double g0 = ppm_g(0, X, d0), g1 = ppm_g(1, X, d1), g2 = ppm_g(2, X, d2);
+      const double da = g0 * (g1 * dp_ + g2 * dm_);
+      const bool bsel = 2.0 * fabs(dm_) < 2.0 * fabs(dp_);
+      const double bc = bsel ? 2.0 * fabs(dm_) : 2.0 * fabs(dp_);
+      const bool asel = fabs(da) < bc;
+      const double sda = da > 0.0 ? 1.0 : da < 0.0 ? -1.0 : 0.0;
+      const double lm3 = f.F(RF_LDMA, j) * sda;
+      double lda = 0.0;
+      if (asel) {
+        lda = lm3 * sda;
+      } else if (bsel) {
+        ldm = 2.0 * (dm_ > 0.0 ? 1.0 : dm_ < 0.0 ? -1.0 : 0.0) * lm3;
+      } else {
+        ldp = 2.0 * (dp_ > 0.0 ? 1.0 : dp_ < 0.0 ? -1.0 : 0.0) * lm3;
       }
-      LA(j + 1) += c1 + ldp;
-      c1 = c2 + (ldm - ldp);
-      c2 = -ldm;
+      const double lg0 = lda * (g1 * dp_ + g2 * dm_), lg1 = lda * g0 * dp_, lg2 = lda * g0 * dm_;
+      ldp += lda * g0 * g1;
+      ldm += lda * g0 * g2;
+      for (int m = 0; m < 3; ++m) w[m] += lg0 * d0[m] + lg1 * d1[m] + lg2 * d2[m];
     }
-    LA(0) += c1;
-    LA(-1) += c2;
-    for (int m = 0; m < 3; ++m) F(RF_LD, m) += w[m];
+    if (f.own(j + 1)) f.LA(j + 1) += c1 + ldp;
+    c1 = c2 + (ldm - ldp);
+    c2 = -ldm;
   }
-  // ghosts of a fold back; a = var/dx, var = f*dx
-  for (int k = 0; k < L; ++k) {
-    double lao = LA(k + 1);
-    if (k == 0) lao += LA(0);
-    if (k == 1) lao += LA(-1);
-    if (k == L - 1) lao += LA(L + 1);
-    if (k == L - 2) lao += LA(L + 2);
-    const double x = src(k), fv = fin[fidx(k)], var = fv * x;
-    const double lvar = F(RF_LMASS, k) + lao / x;
-    F(RF_LDX, k) += -lao * var / (x * x) + lvar * fv;
-    lam[fidx(k)] = lvar * x;
+  if (f.chunk == 0) {
+    f.LA(0) += c1;
+    f.LA(-1) += c2;
+  }
+#pragma unroll
+  for (int m = 0; m < 3; ++m)
+    if (f.own(last + m)) f.F(RF_LD, last + m) += w[m];
+}
+
+// ghosts of a fold back; a = var/dx, var = f*dx
+__global__ __launch_bounds__(256) void adj_remap_value_kernel(AdjRemapArgs a) {
+  RField f;
+  if (!remap_lane(a, f)) return;
+  const int L = f.L;
+  for (int k = f.i0; k < f.i1 && k < L; ++k) {
+    double lao = f.LA(k + 1);
+    if (k == 0) lao += f.LA(0);
+    if (k == 1) lao += f.LA(-1);
+    if (k == L - 1) lao += f.LA(L + 1);
+    if (k == L - 2) lao += f.LA(L + 2);
+    const double x = f.src(k), fv = f.fin[f.fidx(k)], var = fv * x;
+    const double lvar = f.F(RF_LMASS, k) + lao / x;
+    f.F(RF_LDX, k) += -lao * var / (x * x) + lvar * fv;
+    f.lam[f.fidx(k)] = lvar * x;
   }
 }
 
@@ -873,19 +1020,34 @@ __global__ __launch_bounds__(256) void adj_remap_finish_kernel(AdjRemapArgs a) {
   double spio = sum3(RF_LPIO, L) + sum3(RF_LPIO, L + 1) + sum3(RF_LPIN, L);
   double spin = 0.0, lps = a.l_ps[col];
   double *ldp = a.l_dp + (size_t)ie * L * 16 + pt;
-  for (int k = L - 1; k >= 0; --k) {
-    // dx(k) enters pio(i) for i > k, the ghosts and ps
-    double x = sum3(RF_LDX, k) + sum3(RF_LD, k + 2) + spio;
-    if (k == 1) x += sum3(RF_LD, 0);
-    if (k == 0) x += sum3(RF_LD, 1);
-    if (k == L - 1) x += sum3(RF_LD, L + 2);
-    if (k == L - 2) x += sum3(RF_LD, L + 3);
-    ldp[(size_t)k * 16] = x;
-    spio += sum3(RF_LPIO, k);
-    // tg(k) enters pin(i) for k < i <= L-1
-    const double ltg = sum3(RF_LTG, k) + spin;
-    spin += sum3(RF_LPIN, k);
-    lps += (a.hybi[k + 1] - a.hybi[k]) * ltg;
+  // (four levels' loads ahead of the stores, which may alias them)
+  for (int b = L - 1; b >= 0; b -= 4) {
+    double xs[4], pio[4], tgs[4], pin[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int k = b - i > 0 ? b - i : 0;
+      xs[i] = sum3(RF_LDX, k) + sum3(RF_LD, k + 2);
+      pio[i] = sum3(RF_LPIO, k);
+      tgs[i] = sum3(RF_LTG, k);
+      pin[i] = sum3(RF_LPIN, k);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int k = b - i;
+      if (k < 0) break;
+      // dx(k) enters pio(i) for i > k, the ghosts and ps
+      double x = xs[i] + spio;
+      if (k == 1) x += sum3(RF_LD, 0);
+      if (k == 0) x += sum3(RF_LD, 1);
+      if (k == L - 1) x += sum3(RF_LD, L + 2);
+      if (k == L - 2) x += sum3(RF_LD, L + 3);
+      ldp[(size_t)k * 16] = x;
+      spio += pio[i];
+      // tg(k) enters pin(i) for k < i <= L-1
+      const double ltg = tgs[i] + spin;
+      spin += pin[i];
+      lps += (a.hybi[k + 1] - a.hybi[k]) * ltg;
+    }
   }
   for (int k = 0; k < L; ++k) ldp[(size_t)k * 16] += lps;
 }
@@ -927,7 +1089,13 @@ void launch_adj_remap(hipStream_t st, const AdjRemapArgs &a) {
   while (gbs > 1 && (size_t)(a.nlev + 2) * gbs * sizeof(double) > 65536) gbs >>= 1;
   hipLaunchKernelGGL(adj_remap_grid_kernel, dim3(nblk(ncol, gbs)), dim3(gbs), (size_t)(a.nlev + 2) * gbs * sizeof(double),
                      st, a);
-  hipLaunchKernelGGL(adj_remap_field_kernel, dim3(nblk(3 * ncol)), dim3(256), 0, st, a);
+  const unsigned nb = nblk(3 * ncol), nc = (unsigned)adj_chunks(a.nlev);
+  hipLaunchKernelGGL(adj_remap_forward_kernel, dim3(nb, nc + 1), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(adj_remap_target_kernel, dim3(nb, nc), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(adj_remap_cell_kernel, dim3(nb, nc + 1), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(adj_remap_interface_kernel, dim3(nb, nc), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(adj_remap_slope_kernel, dim3(nb, nc), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(adj_remap_value_kernel, dim3(nb, nc), dim3(256), 0, st, a);
   hipLaunchKernelGGL(adj_remap_finish_kernel, dim3(nblk(ncol)), dim3(256), 0, st, a);
 }
 size_t adj_remap_scratch(int nelem, int nlev) {
