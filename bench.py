@@ -56,29 +56,29 @@ def kernel_bytes(name, nelem, nlev, q, launches):
     ql = q / 8.0
     if name == "euler_advect":
         # reads Qdp(Q), derived_dp, divdp_proj, vn0(2), divdp, fdss, qlim; writes qdp_pre(Q), fdss_pre.
-        # Stage 2 also writes qlim; it reads stage 1's pre-exchange buffers (Q + 1) in place of the
-        # assembled Qdp and divdp_proj and writes the assembled divdp_proj (its exchange is fused in).
-        # Stage 3 also reads qbih(Q) and dpdiss_bih.
+        # Stage 2 reads stage 1's pre-exchange buffers (Q + 1) in place of the assembled Qdp and
+        # divdp_proj and writes the assembled divdp_proj (it gathers the exchange itself).
+        # Stage 3 also reads the first laplacian (Q) and dpdiss_bih.
         s1 = (q + 6 + ql) + (q + 1)
-        s2 = s1 + ql + 2
+        s2 = s1 + 1
         s3 = s1 + q + 1
         return (s1 + s2 + s3) / 3.0 * F
+    if name == "euler_dss_lap":
+        # stage 2's qdp_pre(Q) + fdss_pre, derived_dp, divdp_proj, dpdiss_ave in; Qdp(Q) + fdss, the
+        # first laplacian (Q) and qlim out
+        return (3 * q + 5 + ql) * F
     if name == "euler_dss":
-        # two launches (stages 2 and 3): qdp_pre(Q) + fdss_pre in, Qdp(Q) + fdss out; stage 3 also
-        # reads Qdp(n0)(Q) for the average
-        s1 = 2 * q + 2
-        return (2 * s1 + q) / 2.0 * F
-    if name == "euler_qmm_lap":
-        # Qdp(Q), derived_dp, divdp_proj, dpdiss_ave in; qbih_pre(Q), qlim out
-        return (2 * q + 3 + ql) * F
-    if name == "euler_bih_post":
-        return 2 * q * F
+        # stage 3's qdp_pre(Q) + fdss_pre and Qdp(n0)(Q) in, Qdp(Q) + fdss out
+        return (3 * q + 2) * F
     if name == "euler_divdp_qmm":
         return (q + 3 + 2 + ql) * F
     if name == "caar":
-        return (10 + 3 + 1 + 4) * F  # reads n0(4), nm1(4), vn0(2), omega; writes 4, vn0(2), omega, phi
+        # five stages: the input (4; gathered but for the first) and the output (4); stages 2 to 5 add
+        # to u0 (4); stage 5 also reads u1 (4), writes the combination (4); 1 and 5 accumulate
+        # vn0 (2 + 2) and omega (1 + 1)
+        return (14 + 3 * 12 + 26) / 5.0 * F
     if name == "caar_dss":
-        return 8 * F
+        return 12 * F  # the last stage's output (4) in, the state and its first laplacians out
     if name == "remap":
         return ((3 + q) * 2 + 1 + q) * F  # v,T,Qdp in/out, dp3d, Q out
     return None
