@@ -1,5 +1,5 @@
 // Dynamics right-hand side and update for one RK stage (CAAR), plus the
-// small element-wise kernels of the step (dp3d from ps, prim_step init).
+// small element-wise kernels of the step (dp3d from ps).
 //
 // A block is one element; a lane holds GLL point pt at CL (4 or 6) consecutive
 // levels of it, so the 16 lanes of one group form a slab at each of its
@@ -150,9 +150,15 @@ __global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(MAXT > 512
   // ---------------------------------------------------------------- A
   // (a stage of weight 0 leaves the accumulators alone; stages 2 to 4 have none)
   const bool acc = eta != 0.0;
+  // the first stage of a step starts them and keeps its dp (a launch that cleared
+  // them first cost 16 us of the step at 1536 elements L72, 73 at 5400, and as
+  // many bytes again where they were read back)
+  const bool start = BASE == 0 && a.derived_dp;
   if (on) {
     double q0[CL], q1[CL];
-    if (acc) {
+#pragma unroll
+    for (int j = 0; j < CL; ++j) q0[j] = q1[j] = 0.0;
+    if (acc && !start) {
 #pragma unroll
       for (int j = 0; j < CL; ++j) {
         q0[j] = (a.vn0 + vE)[vi(j)];
@@ -169,6 +175,7 @@ __global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(MAXT > 512
         (a.vn0 + vE)[vi(j)] = q0[j] + eta * vdp0;
         (a.vn0 + vE)[vi(j) + 16] = q1[j] + eta * vdp1;
       }
+      if (start && k0 + j < L) (a.derived_dp + sE)[si(j)] = dp[j];
       sp[(k0 + j) * 16] = dp[j];
       sd[(k0 + j) * 16] = sph_div(e, d, vdp0, vdp1);
     }
@@ -254,14 +261,14 @@ __global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(MAXT > 512
       base_tdp(j + 1);
       const double p = sp[k * 16], integ = ss[k * 16], dv = sd[k * 16];
       const double tvj = MOIST ? tv[j] : t[j];
-      const double om0 = acc ? (a.omega + sE)[si(j)] : 0.0;
+      const double om0 = acc && !start ? (a.omega + sE)[si(j)] : 0.0;
       double tva = 0.0, ek1 = 0.0;
       if (RS0) {
         ek[j] = eta_of(k, integ);
         ek1 = eta_of(k + 1, integ + dv);
         ek[j + 1] = ek1;
         tva = vadv(j ? t[j - 1] : tm, t[j], j + 1 < CL && k + 1 < L ? t[j + 1] : tp, k, dp[j], ek[j], ek1);
-        if (acc && k < L) (a.eta_acc + sE)[si(j)] += eta * ek[j];
+        if (acc && k < L) (a.eta_acc + sE)[si(j)] = (start ? 0.0 : (a.eta_acc + sE)[si(j)]) + eta * ek[j];
       }
       double gp0, gp1;
       sph_grad(e, d, p, gp0, gp1);
@@ -427,32 +434,6 @@ void launch_dp3d_from_ps(hipStream_t st, int nelem, int nlev, const double *hyai
   const size_t n = (size_t)nelem * nlev * 16;
   hipLaunchKernelGGL(dp3d_from_ps_kernel, dim3((n + 255) / 256), dim3(256), 0, st, nelem, nlev, hyai, hybi, ps0, ps,
                      dp);
-}
-
-__global__ void prim_step_init_kernel(size_t n, bool zero_diss, const double *__restrict__ dp_n0,
-                                      double *__restrict__ eta_dot, double *__restrict__ vn0,
-                                      double *__restrict__ omega, double *__restrict__ dpa, double *__restrict__ dpb,
-                                      double *__restrict__ derived_dp) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  eta_dot[i] = 0;
-  omega[i] = 0;
-  const size_t row = i >> 4, pt = i & 15;
-  vn0[row * 32 + pt] = 0;
-  vn0[row * 32 + 16 + pt] = 0;
-  if (zero_diss) {
-    dpa[i] = 0;
-    dpb[i] = 0;
-  }
-  derived_dp[i] = dp_n0[i];
-}
-
-void launch_prim_step_init(hipStream_t st, int nelem, int nlev, bool zero_diss, const double *dp_n0,
-                           double *eta_dot, double *vn0, double *omega, double *dpa, double *dpb,
-                           double *derived_dp) {
-  const size_t n = (size_t)nelem * nlev * 16;
-  hipLaunchKernelGGL(prim_step_init_kernel, dim3((n + 255) / 256), dim3(256), 0, st, n, zero_diss, dp_n0, eta_dot,
-                     vn0, omega, dpa, dpb, derived_dp);
 }
 
 }  // namespace hx

@@ -359,6 +359,7 @@ struct StateBuf {
 struct RkBufs {
   StateBuf u[5], w, out;
   bool keep = false;
+  bool start = false;  // the accumulators start here
 };
 
 StateBuf level(int tl) {
@@ -448,6 +449,7 @@ void rk_stages(const RkBufs &r, double dt, double eta_ave_w) {
     a.pre_out = c.pre[i & 1];
     a.dt = h[i];
     a.eta_ave_w = eta[i];
+    a.derived_dp = i == 0 && r.start ? c.derived_dp : nullptr;
     a.p_top = c.hyai0 * c.ps0;
     {
       Scope s("caar");
@@ -460,8 +462,9 @@ void rk_stages(const RkBufs &r, double dt, double eta_ave_w) {
   state_dss(c.pre[0], r.out, true);
 }
 
-void u3_5stage(int nm1, int n0, int np1, double dt, double eta_ave_w) {
+void u3_5stage(int nm1, int n0, int np1, double dt, double eta_ave_w, bool start) {
   RkBufs r;
+  r.start = start;
   r.u[0] = level(n0);
   r.u[1] = r.w = level(nm1);
   r.u[2] = r.u[3] = r.u[4] = r.out = level(np1);
@@ -502,12 +505,13 @@ HvArgs hv_args(const StateBuf &x, const StateBuf &o, double dt, double eta_ave_w
   return a;
 }
 
-void hyperviscosity(int np1, double dt, double eta_ave_w) {
+void hyperviscosity(int np1, double dt, double eta_ave_w, bool start) {
   Ctx &c = C();
-  const HvArgs a = hv_args(level(np1), level(np1), dt, eta_ave_w);
+  HvArgs a = hv_args(level(np1), level(np1), dt, eta_ave_w);
   const int nsub = c.p.hypervis_subcycle;
   for (int cyc = 0; cyc < nsub; ++cyc) {
     Scope s("hv_cycle");
+    a.first = start && cyc == 0;
     launch_hv_cycle(c.st, a, cyc + 1 < nsub);
   }
 }
@@ -625,18 +629,16 @@ void advec_tracers(double dt) {
 
 void prim_step(double dt) {
   Ctx &c = C();
-  {
-    Scope s("prim_step_init");
-    launch_prim_step_init(c.st, c.nelem, c.nlev, c.p.nu_p > 0, c.dp[c.n0], c.eta_dot, c.vn0, c.omega, c.dpdiss_ave,
-                          c.dpdiss_bih, c.derived_dp);
-  }
+  // The accumulators (vn0, omega, eta_dot, the dissipation) and the derived dp
+  // start in the first dynamics step's first stage and first subcycle.  (With
+  // rsplit > 0 nothing adds to eta_dot: it keeps the zeros it is allocated with.)
   for (int n = 0; n < c.p.qsplit; ++n) {
     if (n > 0) leapfrog();
     if (c.p.moist) update_tracers_levels();
     const double eta_ave_w = 1.0 / c.p.qsplit;
-    u3_5stage(c.nm1, c.n0, c.np1, dt, eta_ave_w);
+    u3_5stage(c.nm1, c.n0, c.np1, dt, eta_ave_w, n == 0);
     if (c.stopped || stop_here(2)) return;
-    hyperviscosity(c.np1, dt, eta_ave_w);
+    hyperviscosity(c.np1, dt, eta_ave_w, n == 0 && c.p.nu_p > 0);
     if (stop_here(3)) return;
   }
   if (c.qsize > 0) advec_tracers(dt * c.p.qsplit);

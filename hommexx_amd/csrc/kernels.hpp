@@ -32,6 +32,7 @@ struct CaarArgs {
   const double *hybi;           // nlev+1 interface b coefficients (rsplit == 0)
   double *eta_acc;              // eta_dot_dpdn accumulator (rsplit == 0)
   double *pre_out;              // pre-exchange result [ie][4][sc]
+  double *derived_dp;                // set: the accumulators start here, dp is kept in it
   double dt, eta_ave_w, p_top;  // p_top = hyai(0)*ps0
 };
 
@@ -190,8 +191,6 @@ void launch_adj_ps(hipStream_t st, int nelem, int nlev, const double *hybi, cons
 void launch_adj_zero(hipStream_t st, size_t n, double *p);
 void launch_dp3d_from_ps(hipStream_t st, int nelem, int nlev, const double *hyai_d, const double *hybi_d, double ps0,
                          const double *ps, double *dp);
-void launch_prim_step_init(hipStream_t st, int nelem, int nlev, bool zero_diss, const double *dp_n0,
-                           double *eta_dot, double *vn0, double *omega, double *dpa, double *dpb, double *derived_dp);
 void launch_caar(hipStream_t st, const CaarArgs &a);
 void launch_dss(hipStream_t st, const DssArgs &a);
 void launch_state_dss(hipStream_t st, const StateDssArgs &a);
