@@ -74,9 +74,9 @@ def kernel_bytes(name, nelem, nlev, q, launches):
         return (q + 3 + 2 + ql) * F
     if name == "caar":
         # five stages: the input (4; gathered but for the first) and the output (4); stages 2 to 5 add
-        # to u0 (4); stage 5 also reads u1 (4), writes the combination (4); 1 and 5 accumulate
-        # vn0 (2 + 2) and omega (1 + 1)
-        return (14 + 3 * 12 + 26) / 5.0 * F
+        # to u0 (4); stage 1 writes vn0 (2), omega and the derived dp; stage 5 also reads u1 (4),
+        # writes the combination (4) and adds to vn0 (2 + 2) and omega (1 + 1)
+        return (12 + 3 * 12 + 26) / 5.0 * F
     if name == "caar_dss":
         return 12 * F  # the last stage's output (4) in, the state and its first laplacians out
     if name == "remap":
