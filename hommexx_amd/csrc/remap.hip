@@ -119,8 +119,10 @@ __device__ __forceinline__ void ppm_parabola(double al, double ar, double a, dou
 // cell kid that holds its lower interface, the offset z2 in it and the
 // reciprocal target thickness.  The thickness sums are serial scans by the
 // first 16 lanes; each (target, column) then searches by itself, from the
-// interface of its own level (the sums grow, so the reference's search, which
-// goes on from the last target's interface, ends at the same one).
+// interface of its own level.  remap_kernel's search goes on from the last
+// target's cell, which is the same unless a target interface lies above the one
+// before (ps fell so far that the target thickness is negative): then the first
+// 16 lanes take the cells down their columns again.
 //
 // Bound: the latency of a block's chain, about 8 us of tables and 10 us a round
 // of fields (one block of 8 or 12 waves fills a CU's LDS).
@@ -149,10 +151,11 @@ __device__ __forceinline__ void unrolled(F &&f) {
 __device__ __forceinline__ double sel3(int i, double a, double b, double c) { return i == 0 ? a : i == 1 ? b : c; }
 
 // One field of one column, top to bottom (fac: the row of Fortran cell -2).
-// A source level is read before its target is written: cell c's parabola
-// needs levels up to c+2, and the targets found in cells up to c are at most c.
+// In place: when the targets of cell c (at most c+1) are written, the levels that
+// later cells' parabolas need are in registers up to level c+2 (A2), read before.
+// kid does not decrease, so each target is met.  Returns whether all were.
 template <typename Put>
-__device__ __forceinline__ void remap_column(const double *fac, const double *zsh, const short *ksh, int L, int alg,
+__device__ __forceinline__ bool remap_column(const double *fac, const double *zsh, const short *ksh, int L, int alg,
                                              const double *var, unsigned vs, bool state, Put put) {
   auto row = [&](int j) { return fac + (j + 2) * RG2 * 16; };
   auto mirror = [&](int r) { return r < 0 ? -r - 1 : r >= L ? 2 * L - 1 - r : r; };
@@ -199,6 +202,7 @@ __device__ __forceinline__ void remap_column(const double *fac, const double *zs
     dma0 = dma1;
     ai_prev = ai;
   }
+  return k == L;
 }
 
 template <int N, int FB>
@@ -216,6 +220,7 @@ __global__ __launch_bounds__(FB == 1 ? 768 : 512) void remap_split_kernel(RemapA
   double *const dab = rtk + L4 * 16;                    // hyai(k+1) - hyai(k), hybi(k+1) - hybi(k)  [L4][2]
   double *const pss = dab + L4 * 2;                     // ps [16]
   int *const deep = (int *)(pss + 16);                  // a target lies in none of its three cells
+  int *const back = deep + 1;                           // a target interface lies above the one before
   short *const ksh = (short *)(deep + 4);               // kid [L4][16]
   double *const dxs = rtk;                              // first the source thicknesses
   const int ie = xcd_block(blockIdx.x, gridDim.x);
@@ -238,7 +243,7 @@ __global__ __launch_bounds__(FB == 1 ? 768 : 512) void remap_split_kernel(RemapA
       ksh[i] = (short)(i >> 4);
       zsh[i] = 0.0;
     }
-    if (tid == 0) *deep = 0;
+    if (tid == 0) *deep = *back = 0;
     if (bad) atomicOr(a.error, 1);
   }
   __syncthreads();
@@ -312,9 +317,27 @@ __global__ __launch_bounds__(FB == 1 ? 768 : 512) void remap_split_kernel(RemapA
     zsh[i] = kid >= 0 ? (pk - (pio[kid * 16 + p] + pio[si * 16 + p]) * 0.5) / fac[((kid + 3) * RG2 + 8) * 16 + p] : 0.0;
     rtk[i] = 1.0 / target(k, pss[p]);
     if (kid > k + 1) *deep = 1;
+    if (k > 0 && pk < pin[k * 16 + p]) *back = 1;
     if (kid < 0) atomicOr(a.error, 2);  // below the first interface: not a column the reference remaps
   }
   __syncthreads();
+  if (*back) {
+    if (tid < 16) {
+      int last = 0;
+      for (int k = 0; k < L; ++k) {
+        const int i = k * 16 + tid, kid = ksh[i];
+        if (kid >= last) {
+          last = kid;
+        } else if (k > 0) {
+          ksh[i] = (short)last;
+          zsh[i] = (pin[i + 16] - (pio[last * 16 + tid] + pio[(last + 1) * 16 + tid]) * 0.5) /
+                   fac[((last + 3) * RG2 + 8) * 16 + tid];
+          if (last > k + 1) *deep = 1;
+        }
+      }
+    }
+    __syncthreads();
+  }
 
   // ------------------------------------------------------------ fields
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = nt >> 6;
@@ -364,9 +387,10 @@ __global__ __launch_bounds__(FB == 1 ? 768 : 512) void remap_split_kernel(RemapA
     if (general) {
 #pragma unroll
       for (int b = 0; b < FB; ++b)
-        if (grp == 0 && on[b])
-          remap_column(fg, zg, kg, L, a.remap_alg, var[b] + pt, vs[b], state[b],
-                       [&](int i, double out) { put(b, i, out, thickness(i)); });
+        if (grp == 0 && on[b] &&
+            !remap_column(fg, zg, kg, L, a.remap_alg, var[b] + pt, vs[b], state[b],
+                          [&](int i, double out) { put(b, i, out, thickness(i)); }))
+          atomicOr(a.error, 2);
       continue;
     }
     // levels c0-3 .. c0+n+2, all in registers before the first store
