@@ -902,14 +902,14 @@ void hv_adjoint(AdjBufs &b, const StateBuf &x, const StateBuf &xo, const StateBu
 
 // Copies between device arrays and rows of host arrays (rows of `row` doubles,
 // `stride` apart on the host, adjacent on the device), made when the object goes
-// out of scope: nothing is left to do after that.  They run in pieces through
-// pinned buffers, on up to HostStage::W threads with two buffers each, the
-// transfer of one piece beside the host's copy of others.  A copy to or from
-// pageable memory runs at 18 and 31-37 GB/s and needs a contiguous host copy
-// first; a pinned one runs at 56 GB/s, one thread's copy between a buffer and the
-// rows at 20-30.  A physics interval at 384 elements L72 Q4 (141 MB both ways,
-// six steps) took 17.7 ms with the former, 8.9 through one thread, 7.1
-// through four (7.6 two; pieces of 1 MB 8.3, of 4 MB 7.0).
+// out of scope (or MAX_ARRAYS are pending): nothing is left to do after that.
+// They run in pieces through pinned buffers, on up to HostStage::W threads with
+// two buffers each, the transfer of one piece beside the host's copy of others.
+// A copy to or from pageable memory runs at 18 and 31-37 GB/s and needs a
+// contiguous host copy first; a pinned one runs at 56 GB/s, one thread's copy
+// between a buffer and the rows at 20-30.  A physics interval at 384 elements L72
+// Q4 (141 MB both ways, six steps) took 17.7 ms with the former, 8.9 through one
+// thread, 7.1 through four (7.6 two; pieces of 1 MB 8.3, of 4 MB 7.0).
 class HostCopy {
  public:
   explicit HostCopy(bool to_host) : c_(C()), to_host_(to_host), lock_(stage_mutex()) {}
@@ -923,8 +923,19 @@ class HostCopy {
     const size_t e3 = (size_t)c_.nlev * 16;
     add(dev, host + (size_t)tl * c_.qsize_d * e3, (size_t)c_.qsize * e3, (size_t)ntl * c_.qsize_d * e3);
   }
-  ~HostCopy() {
+  ~HostCopy() { run(); }
+
+ private:
+  // what is pending, to its end
+  void run() {
     if (!npieces_) return;
+    copy();
+    narrays_ = 0;
+    npieces_ = total_ = 0;
+    taken_ = 0;
+    error_ = hipSuccess;
+  }
+  void copy() {
     // (a thread for every 8 MB)
     const size_t share = total_ / (4 * HostStage::PIECE);
     const int n = std::max(1, (int)std::min<size_t>({(size_t)HostStage::W, std::thread::hardware_concurrency(), share}));
@@ -953,8 +964,6 @@ class HostCopy {
     const hipError_t es = hipStreamSynchronize(c_.st);
     hipok(e != hipSuccess ? e : es, "host copy");
   }
-
- private:
   static std::mutex &stage_mutex() {
     static std::mutex m;
     return m;
@@ -967,6 +976,7 @@ class HostCopy {
   void add(double *dev, const double *host, size_t row, size_t stride) {
     const size_t n = (size_t)c_.nelem * row;
     if (!n) return;
+    if (narrays_ == MAX_ARRAYS) run();
     // (the host's rows are written only where to_host_)
     arrays_[narrays_++] = Array{dev, const_cast<double *>(host), row, stride, n, npieces_};
     npieces_ += (n + HostStage::PIECE - 1) / HostStage::PIECE;
