@@ -829,9 +829,21 @@ void launch_ps_from_dp(hipStream_t st, int nelem, int nlev, double hyai0, double
 //                  43 2319/1981; L40 15 fields 624/545, L26 15 fields 440/365
 //   few elements:  ne4 L26 7 fields 17/52, 43 51/76; ne8 L72 43 217/253, L26 43
 //                  104/102; ne11 (726 elements) L26 43 157/129
+// Below 20 levels the chain that is split is short, and a wave's slopes and
+// tables ahead of its first target (4 + 4 steps whatever the run) weigh more:
+//   3 to 8 levels: ne30 L3 8 fields 140/54, L6 162/82; ne16 L5 6 fields 48/29; ne8
+//                  L6 8 fields 19/22, 15 fields 28/23; ne11 4 fields 15/21
+//   12 levels:     ne16 6 fields 55/51, ne11 8 fields 32/37, ne30 4 fields 88/105
+//   16, 17 levels: ne16 8 fields 61/76; ne24 8 fields L17 144/143; ne30 8 fields L17
+//                  219/202, 4 fields 109/175
+// (a block has four waves at least, so fewer fields cost it what four do).
 constexpr int REMAP_SPLIT_ELEMS = 512;  // two blocks per CU
 static bool remap_split(int nelem, int nlev, int nfld) {
   if (nlev > REMAP_SPLIT_NLEV || nfld == 0) return false;
+  if (nlev < 20 && !(nfld <= 4 && nlev >= 8)) {
+    const int waves = nlev >= 16 ? 28000 : nlev >= 12 ? 7000 : 4000;
+    if ((long long)nelem * (nfld < 4 ? 4 : nfld) > waves) return false;
+  }
   return nfld <= 8 || (nlev > 64 && nfld <= 24) || nelem <= REMAP_SPLIT_ELEMS;
 }
 
