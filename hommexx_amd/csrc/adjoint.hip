@@ -612,13 +612,15 @@ __global__ __launch_bounds__(64) void adj_remap_grid_kernel(AdjRemapArgs a) {
   pio_s[L * bs + tid] = pioL;
   pio_s[(L + 1) * bs + tid] = pioL + 1.0;
   double pin = 0.0;  // pin(k+1), the same running sum as above
+  // the forward search: from interface k, or on from the last target's (which is
+  // further down only where a target thickness is negative), so kid never falls
+  int si = 0;
   for (int k = 0; k < L; ++k) {
     pin += (a.hyai[k + 1] - a.hyai[k]) * a.ps0 + (a.hybi[k + 1] - a.hybi[k]) * ps;
     const double pk = k + 1 < L ? pin : pioL;
-    int kk = k + 1;
-    while (kk - 1 <= L + 1 && pio_s[(kk - 1) * bs + tid] <= pk) kk++;
-    kk--;
-    if (kk == L + 1) kk = L;
+    if (si < k) si = k;
+    while (si <= L + 1 && pio_s[si * bs + tid] <= pk) ++si;
+    const int kk = si >= L + 1 ? L : si;
     // kid >= 0 for every valid column (pio(0) = 0 <= pin(1)); the clamp keeps
     // the reads in bounds for a column the forward step rejected (NaN)
     const int kid = kk - 1 < 0 ? 0 : kk - 1;
