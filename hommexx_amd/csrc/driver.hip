@@ -91,13 +91,12 @@ struct Ctx {
   std::vector<double> qdp_tail;  // Qdp of tracers qsize..qsize_d-1 as received (never evolved)
   std::vector<double> fq_tail;   // FQ of tracers qsize..qsize_d-1 as received (never used)
   // derived
-  double *phi = nullptr, *omega = nullptr, *eta_dot = nullptr, *dpdiss_ave = nullptr, *dpdiss_bih = nullptr,
+  double *omega = nullptr, *eta_dot = nullptr, *dpdiss_ave = nullptr, *dpdiss_bih = nullptr,
          *derived_dp = nullptr, *divdp = nullptr, *divdp_proj = nullptr, *vn0 = nullptr;
   // forcing
   double *ft = nullptr, *fm = nullptr, *fq = nullptr;
   // scratch
   double *pre[2] = {};   // pre-exchange states [ie][4][sc] (state_chunk)
-  double *cdiv = nullptr;
   double *qdp_pre = nullptr, *qlim[2] = {}, *fdss_pre = nullptr;
   // stage-2 pre-exchange buffers: qdp_pre2 and an alias of
   // pre[0], which is free during the tracer step
@@ -323,12 +322,10 @@ bool ready(const char *who) {
 void alloc_work() {
   Ctx &c = C();
   if (c.be_set) return;
-  const size_t e3 = (size_t)c.nelem * c.nlev * 16;
   // pre-exchange buffers: whole 8-level chunks per element and field
   const size_t e3c = (size_t)c.nelem * lc_field(c.nlev), q3c = e3c * (c.qsize ? c.qsize : 1);
   const size_t sc = c.nelem * std::max(sc_field<4>(c.nlev), sc_field<6>(c.nlev));
   for (double *&p : c.pre) p = dalloc<double>(std::max(4 * sc, e3c));
-  c.cdiv = dalloc<double>(e3);
   // Four 40-F3 tracer uses share two allocations (at Q = 40); no kernel
   // writes the allocation it gathers from:
   //   qdp_pre : stage-1 pre-exchange (-> stage 2), then the first laplacian of
@@ -652,7 +649,7 @@ void remap(double dt_remap) {
   a.qsize = c.qsize;
   a.nstates = c.p.rsplit > 0 ? 3 : 0;
   a.eta = c.eta_dot;
-  a.src = c.cdiv;  // CAAR's scratch is free at the remap
+  a.src = c.pre[0];  // free at the remap
   a.dt = dt_remap;
   a.remap_alg = c.p.remap_alg;
   a.v = c.v[c.np1];
@@ -1545,7 +1542,6 @@ void init_elements_2d_c(const int &num_elems, const double *const &D, const doub
   }
   for (int tl = 0; tl < 2; ++tl) c.qdp[tl] = dalloc<double>(e3 * (c.qsize ? c.qsize : 1));
   c.Q = dalloc<double>(e3 * (c.qsize ? c.qsize : 1));
-  c.phi = dalloc<double>(e3);
   c.omega = dalloc<double>(e3);
   c.eta_dot = dalloc<double>(e3);
   c.dpdiss_ave = dalloc<double>(e3);

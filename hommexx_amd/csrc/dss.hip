@@ -24,31 +24,6 @@ __global__ __launch_bounds__(256) void dss_kernel(DssArgs a) {
   auto at = [&](const DssField &F, int src, size_t own) {
     return opaque_index(src >= 0 ? (size_t)(src >> 4) * F.estride + (size_t)k * F.lstride + (src & 15) : own);
   };
-  if (a.f32) {
-    // FP32 fields of the mixed form, accumulated in FP64
-    float r[DSS_MAX_FIELDS][4];
-#pragma unroll
-    for (int f = 0; f < DSS_MAX_FIELDS; ++f) {
-      if (f < a.nf) {
-        const DssField &F = a.f[f];
-        const float *in = (const float *)F.in;
-        const size_t own = (size_t)ie * F.estride + (size_t)k * F.lstride + pt;
-        r[f][0] = in[own];
-        r[f][1] = in[at(F, s0, own)];
-        r[f][2] = in[at(F, s1, own)];
-        r[f][3] = in[at(F, s2, own)];
-      }
-    }
-#pragma unroll
-    for (int f = 0; f < DSS_MAX_FIELDS; ++f) {
-      if (f < a.nf) {
-        const DssField &F = a.f[f];
-        const double x = gather_sum(r[f], s0, s1, s2);
-        ((float *)F.out)[(size_t)ie * F.estride + (size_t)k * F.lstride + pt] = (float)(a.rsmp ? x * r0 : x);
-      }
-    }
-    return;
-  }
   double r[DSS_MAX_FIELDS][4];
 #pragma unroll
   for (int f = 0; f < DSS_MAX_FIELDS; ++f) {

@@ -60,7 +60,6 @@ struct DssField {
 struct DssArgs {
   DssField f[DSS_MAX_FIELDS];
   int nf, nelem, nlev;
-  int f32;               // fields hold FP32 values (accumulated in FP64)
   const int *src;        // [ie][16][3] global point ids (ie*16 + pt) or -1
   const double *rsmp;    // multiply by rspheremp if non-null
 };
@@ -93,7 +92,6 @@ __host__ __device__ inline size_t lc_index(int pt, int k) { return (size_t)(k >>
 // to a multiple of 8 levels (one 128-byte line per 8 levels).
 __host__ __device__ inline size_t ql_row(int nlev) { return (size_t)((nlev + 7) >> 3) * 16; }
 __host__ __device__ inline size_t ql_min(int k) { return (size_t)k * 2; }
-constexpr int QL_MAX = 1;  // offset of a level's maximum from its minimum
 
 struct EulerArgs {
   MetricPtrs m;

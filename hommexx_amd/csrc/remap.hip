@@ -668,14 +668,13 @@ __global__ __launch_bounds__(256) void remap_kernel(RemapArgs a) {
       const double x0 = var[i][0], x1 = var[i][vs[i]];
       const double v0 = state[i] ? x0 * s0 : x0, v1 = state[i] ? x1 * s1 : x1;
       const double a1 = v0 / s0, a2 = v1 / s1;
-      const double am1 = alg == 3 ? a1 : a2;  // a(-1)
       A0[i] = a1;  // a(0) = a(1)
       A1[i] = a1;
       A2[i] = a2;
       V0[i] = 0.0;
       V1[i] = v0;
       V2[i] = v1;
-      dma_j[i] = ppm_dma_g(am1, A0[i], A1[i], g0, g1, g2);  // dma(0)
+      dma_j[i] = ppm_dma_g(a2, A0[i], A1[i], g0, g1, g2);  // dma(0), a(-1) = a(2)
       ai_prev[i] = 0.0;
       var_prefix[i] = 0.0;
       mass_prev[i] = 0.0;
@@ -786,7 +785,7 @@ __global__ __launch_bounds__(256) void remap_kernel(RemapArgs a) {
         } else if (m == L + 1) {
           an = A2[i];  // a(L+1) = a(L)
         } else {
-          an = alg == 3 ? A1[i] : A0[i];  // a(L+2) = a(L) or a(L-1)
+          an = A0[i];  // a(L+2) = a(L-1)
         }
         A0[i] = A1[i]; A1[i] = A2[i]; A2[i] = an;
         V0[i] = V1[i]; V1[i] = V2[i]; V2[i] = vn;
