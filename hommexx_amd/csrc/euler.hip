@@ -261,7 +261,7 @@ struct WkLds {
 // limiter_optim_iter_full (:767-823), one slab = one level of one tracer
 __device__ __forceinline__ void limit8_slab(double mass, double minp, double maxp, double &x, double c) {
   const double tol_limiter = 5e-14;
-// ( times for two levels: 40 KB of code)
+  // (unrolled 15 times for two levels, it is 40 of a stage's 45 KB of code)
   for (int iter = 0; iter < NP2 - 1; ++iter) {
     double delta = 0;
     if (x > maxp) {

@@ -218,8 +218,9 @@ struct DiagArgs {
 void launch_diag_energy(hipStream_t st, const DiagArgs &a);
 void launch_diag_scalars(hipStream_t st, const DiagArgs &a);
 
-// largest nlev of the remap kernel: an element's target table (10 B per
-// level and column) and a grid chunk (20 KB) fit in 64 KB of LDS
+// The most levels: of 160 KB of LDS a block of remap_kernel then takes 100 KB (304 B
+// a level and a grid chunk of 22 KB), one of CAAR 98 KB, and a block of CAAR has the
+// most lanes there are (1024: 16 for each four levels).
 constexpr int REMAP_MAX_NLEV = 256;
 void launch_remap(hipStream_t st, const RemapArgs &a);
 void launch_ps_from_dp(hipStream_t st, int nelem, int nlev, double hyai0, double ps0, const double *dp, double *ps);
