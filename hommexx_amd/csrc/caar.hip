@@ -1,7 +1,7 @@
 // Dynamics right-hand side and update for one RK stage (CAAR), plus the
 // small element-wise kernels of the step (dp3d from ps).
 //
-// A block is one element; a lane holds GLL point pt at CL (4 or 6) consecutive
+// A block is one element; a lane holds GLL point pt at CL (2, 4 or 6) consecutive
 // levels of it, so the 16 lanes of one group form a slab at each of its
 // levels (cross-lane derivatives) and the whole column's state stays in
 // registers over the phases:
@@ -390,7 +390,7 @@ static void launch_caar_as(hipStream_t st, const CaarArgs &a) {
   // six levels per lane (up to 96 levels: 256 lanes) and rsplit == 0 hold more
   // (168 VGPRs), which blocks of up to 512 lanes may
   constexpr int T = RS0 || CL > 4 ? 512 : 1024;
-  if constexpr (RS0) {
+  if constexpr (RS0 && CL > 2) {
     if (threads.x > T) {
       go(a.qdp_n0 ? caar_kernel<CL, RS0, GATHER, BASE, true, 1024> : caar_kernel<CL, RS0, GATHER, BASE, false, 1024>);
       return;
@@ -406,13 +406,20 @@ static void launch_caar_cl(hipStream_t st, const CaarArgs &a) {
   else launch_caar_as<CL, false, true, 2>(st, a);
 }
 
+template <int CL>
+static void launch_caar_rs0(hipStream_t st, const CaarArgs &a) {
+  if (a.wv) launch_caar_as<CL, true, false, 2>(st, a);
+  else if (a.bv) launch_caar_as<CL, true, false, 1>(st, a);
+  else launch_caar_as<CL, true, false, 0>(st, a);
+}
+
 void launch_caar(hipStream_t st, const CaarArgs &a) {
   if (!a.rsplit0) {
     if (a.chunk == 6) launch_caar_cl<6>(st, a);
+    else if (a.chunk == 2) launch_caar_cl<2>(st, a);
     else launch_caar_cl<4>(st, a);
-  } else if (a.wv) launch_caar_as<4, true, false, 2>(st, a);
-  else if (a.bv) launch_caar_as<4, true, false, 1>(st, a);
-  else launch_caar_as<4, true, false, 0>(st, a);
+  } else if (a.chunk == 2) launch_caar_rs0<2>(st, a);
+  else launch_caar_rs0<4>(st, a);
 }
 
 // ------------------------------------------------------------------ small

@@ -124,6 +124,7 @@ static void launch_state_dss_c(hipStream_t st, const StateDssArgs &a) {
 
 void launch_state_dss(hipStream_t st, const StateDssArgs &a) {
   if (a.chunk == 6) launch_state_dss_c<6>(st, a);
+  else if (a.chunk == 2) launch_state_dss_c<2>(st, a);
   else launch_state_dss_c<4>(st, a);
 }
 
@@ -149,13 +150,17 @@ __global__ __launch_bounds__(256) void hv_lap2_kernel(HvArgs a) {
     if constexpr (TENSOR) return sph_laplace_tensor(o.e, o.d, tv, x);
     else return o.lap(x);
   };
-  const bool top = a.nu_top > 0 && k0 == 0;
+  const bool top = a.nu_top > 0 && k0 < 3;
+  constexpr int TOP = C < 3 ? C : 3;
+  auto top_level = [&](int j) { return C < 3 ? k0 + j : j; };  // (k0 is 0 in longer chunks)
   // the sponge adds sc(j) * (own first laplacian) at levels 0..2
   auto sponge = [&](size_t off, double (&x)[C]) {
     if (!top) return;
 #pragma unroll
-    for (int j = 0; j < 3; ++j)
-      if (j < L) x[j] += (j == 0 ? 4.0 : j == 1 ? 2.0 : 1.0) * a.nu_top * (double)g.p[0][off + j];
+    for (int j = 0; j < TOP; ++j) {
+      const int k = top_level(j);
+      if (k < 3 && k < L) x[j] += (k == 0 ? 4.0 : k == 1 ? 2.0 : 1.0) * a.nu_top * (double)g.p[0][off + j];
+    }
   };
   double *const out = a.pre + (size_t)ie * 4 * lf + (size_t)k0 * 16 + pt * C;
   double x[C], y[C];
@@ -221,11 +226,12 @@ __global__ __launch_bounds__(256) void hv_lap2_kernel(HvArgs a) {
   } else if (top) {
     const size_t v = (size_t)ie * L * 32 + pt;
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      if (j >= L) break;
+    for (int j = 0; j < TOP; ++j) {
+      const int k = top_level(j);
+      if (k >= 3 || k >= L) break;
       P l1;
-      const double l0 = o.vlap(1.0, a.v[v + j * 32], a.v[v + j * 32 + 16], l1);
-      const double sc = (j == 0 ? 4.0 : j == 1 ? 2.0 : 1.0) * a.nu_top;
+      const double l0 = o.vlap(1.0, a.v[v + k * 32], a.v[v + k * 32 + 16], l1);
+      const double sc = (k == 0 ? 4.0 : k == 1 ? 2.0 : 1.0) * a.nu_top;
       x[j] += sc * l0;
       y[j] += sc * (double)l1;
     }
@@ -306,6 +312,7 @@ static void launch_hv_cycle_c(hipStream_t st, const HvArgs &a, bool lap1_next) {
 
 void launch_hv_cycle(hipStream_t st, const HvArgs &a, bool lap1_next) {
   if (a.chunk == 6) launch_hv_cycle_c<6>(st, a, lap1_next);
+  else if (a.chunk == 2) launch_hv_cycle_c<2>(st, a, lap1_next);
   else launch_hv_cycle_c<4>(st, a, lap1_next);
 }
 

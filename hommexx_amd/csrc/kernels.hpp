@@ -431,8 +431,14 @@ __device__ __forceinline__ bool group_slab(int nelem, int nlev, int &ie, int &k,
 // wave slots empty (the dispatcher puts the first and fifth wave of every
 // block on the same SIMD).  CAAR at ne30, per level and step: 15.0 us at 64
 // levels (four waves), 19.2 us at 72 with four levels per lane (five waves).
-// The vertical advection of rsplit == 0 needs the registers.
-inline int state_chunk(int nlev, bool rsplit0) { return !rsplit0 && nlev > 64 && nlev <= 96 ? 6 : 4; }
+// The vertical advection of rsplit == 0 needs the registers.  Two up to 8 levels,
+// where a lane's levels are its chain and the grid leaves units idle: CAAR,
+// exchange and hyperviscosity of a step at 384 elements, 4 levels took 131 us with a
+// lane a level, 148 with four, 106 with two (mixed form 125, 163, 114; rsplit == 0
+// 141, 181, 131).
+inline int state_chunk(int nlev, bool rsplit0) {
+  return nlev <= 8 ? 2 : !rsplit0 && nlev > 64 && nlev <= 96 ? 6 : 4;
+}
 
 // Lane mapping of the other kernels on that layout: a 16-lane group is one
 // element's chunk of levels; elements first, so that neighbour copies come
