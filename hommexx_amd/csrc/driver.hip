@@ -907,6 +907,10 @@ void hv_adjoint(AdjBufs &b, const StateBuf &x, const StateBuf &xo, const StateBu
 // between a buffer and the rows at 20-30.  A physics interval at 384 elements L72
 // Q4 (141 MB both ways, six steps) took 17.7 ms with the former, 8.9 through one
 // thread, 7.1 through four (7.6 two; pieces of 1 MB 8.3, of 4 MB 7.0).
+// What fits one buffer goes through it side by side, with one wait for all: in
+// pieces an array's transfer is waited for every second array.  Initial states and
+// results of 24 elements, 26 levels, 1 tracer: 231 and 260 us in pieces, 194 and
+// 239 from pageable memory, 154 and 217 so.
 class HostCopy {
  public:
   explicit HostCopy(bool to_host) : c_(C()), to_host_(to_host), lock_(stage_mutex()) {}
@@ -936,12 +940,18 @@ class HostCopy {
     // (a thread for every 8 MB)
     const size_t share = total_ / (4 * HostStage::PIECE);
     const int n = std::max(1, (int)std::min<size_t>({(size_t)HostStage::W, std::thread::hardware_concurrency(), share}));
+    HostStage &s = c_.stage;
+    auto pinned = [&](int i) {
+      return s.buf[i] || hipok(hipHostMalloc((void **)&s.buf[i], HostStage::PIECE * sizeof(double)), "hipHostMalloc");
+    };
+    if (total_ <= HostStage::PIECE) {
+      if (pinned(0)) copy_small(s.buf[0]);
+      return;
+    }
     int dev = 0;
     if (!hipok(hipGetDevice(&dev), "host copy")) return;
     for (int i = 0; i < 2 * n; ++i) {
-      HostStage &s = c_.stage;
-      if (!s.buf[i] && !hipok(hipHostMalloc((void **)&s.buf[i], HostStage::PIECE * sizeof(double)), "hipHostMalloc"))
-        return;
+      if (!pinned(i)) return;
       if (!s.ev[i] && !hipok(hipEventCreateWithFlags(&s.ev[i], hipEventDisableTiming), "hipEventCreate")) return;
     }
     std::thread helper[HostStage::W];
@@ -960,6 +970,22 @@ class HostCopy {
     hipError_t e = (hipError_t)error_.load();
     const hipError_t es = hipStreamSynchronize(c_.st);
     hipok(e != hipSuccess ? e : es, "host copy");
+  }
+  // all arrays through one buffer
+  void copy_small(double *buf) {
+    size_t at = 0;
+    for (int k = 0; k < narrays_; at += arrays_[k++].n) {
+      const Array &a = arrays_[k];
+      if (!to_host_) host_copy(a, 0, a.n, buf + at);
+      if (!good(to_host_ ? hipMemcpyAsync(buf + at, a.dev, a.n * sizeof(double), hipMemcpyDeviceToHost, c_.st)
+                         : hipMemcpyAsync(a.dev, buf + at, a.n * sizeof(double), hipMemcpyHostToDevice, c_.st)))
+        break;
+    }
+    const bool done = good(hipStreamSynchronize(c_.st));
+    at = 0;
+    for (int k = 0; k < narrays_ && to_host_ && done && error_.load() == hipSuccess; at += arrays_[k++].n)
+      host_copy(arrays_[k], 0, arrays_[k].n, buf + at);
+    hipok((hipError_t)error_.load(), "host copy");
   }
   static std::mutex &stage_mutex() {
     static std::mutex m;
