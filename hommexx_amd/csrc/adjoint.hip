@@ -642,10 +642,10 @@ __global__ __launch_bounds__(64) void adj_remap_grid_kernel(AdjRemapArgs a) {
 // reaches, in the same order, and stores only its own entries: the same
 // values bit for bit, with a launch per dependence between chunks.  The two mass
 // scans are an extra chunk of the passes beside them.
-// Now, us at 1536 and 384 elements L72: forward 156, 44; targets 209, 57; cells 88,
-// 18; interfaces 100, 25; slopes 73, 26; values 48, 14: 674 and 184 in all.  Chunks
-// of 4, 16 and 24 entries: 725, 666, 659 and 197, 237, 284 (before the scans'
-// loads were batched).
+// Now, us at 1536 and 384 elements L72: forward 156, 40; targets 233, 55; cells 95,
+// 18; interfaces 100, 28; slopes 78, 27; values 47, 14: 708 and 181 in all.  Chunks
+// of 4, 16 and 24 entries, measured before the scans' loads were batched (eight:
+// 674 and 184 in those runs): 725, 666, 659 and 197, 237, 284.
 constexpr int ADJ_CH = 8;
 static int adj_chunks(int nlev) { return (nlev + 4 + ADJ_CH - 1) / ADJ_CH; }
 

@@ -131,7 +131,8 @@ __global__ __launch_bounds__(256) void euler_nbr_minmax_kernel(EulerArgs a) {
 // gathers its own points (no hand-off between lanes, no barrier), and two
 // levels' chains run side by side.  Elements first, then chunks: the waves
 // that run together on an XCD are neighbours at the same tracer, so neighbour
-// copies come from its L2.
+// copies come from its L2.  A last chunk that is not full costs a full one (its
+// padding levels do the last level's work): 26 levels take the time of 32.
 //
 // What bounds them is HBM, if enough waves are in flight: a lane's two FP64
 // chains take 100-130 registers, and the times follow the waves per SIMD which
